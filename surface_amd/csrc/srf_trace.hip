@@ -716,10 +716,11 @@ __device__ __forceinline__ bool sph_traverse(const float4 *__restrict__ nodes,
   return false;
 }
 
-// Closest hit (and plain occlusion) of spheres. kPart selects the
-// wavefronts a launch handles: 0 all, 1 those whose lanes share direction
-// signs (the wavefront traversal; no per-lane stack, so the launch holds
-// more wavefronts per CU), 2 the others (the per-lane traversal). Part 1
+// Closest hit (and plain occlusion) of spheres. kPart selects the lanes a
+// launch handles: 0 all, 1 the groups that share direction signs
+// (walk_groups: the wavefront traversal; no per-lane stack, so the launch
+// holds more wavefronts per CU), 2 the lanes in no group (the per-lane
+// traversal). Part 1
 // followed by part 2 on the same rays gives every ray once.
 template <bool kAny, int kPart>
 __global__ void __launch_bounds__(kTraceBlock)
@@ -727,7 +728,8 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
             const uint32_t *__restrict__ sorted_index, const srf_ray *__restrict__ rays,
             const srf_sphere_prev *__restrict__ prevs, uint32_t n, srf_hit *__restrict__ hits,
             const float *__restrict__ tmax_in, uint32_t *__restrict__ occluded,
-            uint32_t max_nodes, uint32_t nprims, SphSub sub) {
+            uint32_t max_nodes, uint32_t nprims, SphSub sub,
+            const BuildParams *__restrict__ params) {
   constexpr bool kWavePath = !kAny && kPart != 2;
   constexpr bool kLanePath = kPart != 1;
   __shared__ uint32_t stack[kLanePath ? 2 * kTraceStack * kTraceBlock : 1];
@@ -747,11 +749,7 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   float t = FLT_MAX;
   uint32_t best = SRF_NO_PRIM;
   bool occ = false;
-  const uint32_t sb = __builtin_amdgcn_readfirstlane(s.sbits);
-  const bool uniform = __all(s.sbits == sb);
-  if (kPart == 1 && !uniform) return;  // left to part 2
-  if (kPart == 2 && !kAny && uniform) return;  // done by part 1
-  if (kWavePath && uniform) {
+  auto walk = [&](uint64_t mask) {
     // Closest hit once per wavefront, as k_trace_tri_wave: with the lanes'
     // direction signs equal, the reference's order (near child by the split
     // axis's sign, far child pushed, no re-test at the pop) is one static
@@ -759,12 +757,10 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     // traversal visits, holding the distance that traversal would hold
     // there. Small leaves are scanned once per wavefront in the reference's
     // order; a big leaf's secondary tree, whose result does not depend on
-    // its order, runs per lane.
-    t = FLT_MAX;
-    best = SRF_NO_PRIM;
+    // its order, likewise.
+    const uint32_t sb = __builtin_amdgcn_readlane((int)s.sbits, __builtin_ctzll(mask));
     const int wv = threadIdx.x >> 6;
     const uint64_t me = 1ull << (threadIdx.x & 63u);
-    uint64_t mask = __ballot(1);
     uint32_t cur = 0;
     int wsp = 0;
     // the descent's node in scalar registers, both children requested before
@@ -856,10 +852,19 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
       mask = wmask[wv][wsp];
       have = false;
     }
-  } else if constexpr (kLanePath) {
-    occ = sph_traverse<kAny, kTraceBlock>(nodes, prims, sorted_index, max_nodes, nprims, sub, s,
-                                          prev, prevT, prevN, tlimit, stack + threadIdx.x, t,
-                                          best);
+  };
+  int group = -1;
+  if constexpr (!kAny) {
+    group = wave_group(s, group_reach(params));
+    if constexpr (kWavePath) walk_groups(group, walk);
+    if (kPart == 1 && group < 0) return;   // left to part 2
+    if (kPart == 2 && group >= 0) return;  // done by part 1
+  }
+  if constexpr (kLanePath) {
+    if (group < 0)
+      occ = sph_traverse<kAny, kTraceBlock>(nodes, prims, sorted_index, max_nodes, nprims, sub, s,
+                                            prev, prevT, prevN, tlimit, stack + threadIdx.x, t,
+                                            best);
   }
   if (kAny) {
     occluded[i] = occ ? 1u : 0u;
@@ -2178,16 +2183,16 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   const double oj = axis == 0 ? ro.x : (axis == 1 ? ro.y : ro.z);
   const double dj = axis == 0 ? rd.x : (axis == 1 ? rd.y : rd.z);
   uint4 meta;
-  const uint32_t sb = __builtin_amdgcn_readfirstlane(s.sbits);
-  if (!kAny && __all(s.sbits == sb)) {
-    // Closest hit once per wavefront when the lanes' direction signs agree:
+  auto walk = [&](uint64_t group) {
+    // Closest hit once per group of lanes that share direction signs:
     // boxes are culled by entry alone, so a ray's visits do not depend on
     // its running hit and every lane's pre-order is one static order (the
     // line kernel's shared-stack walk); each lane tests its own leaves'
     // solids in its own order, the solids loaded through the scalar unit.
+    const uint32_t sb = __builtin_amdgcn_readlane((int)s.sbits, __builtin_ctzll(group));
     const int wv = threadIdx.x >> 6;
     const uint64_t me = 1ull << (threadIdx.x & 63u);
-    uint64_t mask = __ballot(cur == 0);
+    uint64_t mask = __ballot(cur == 0) & group;
     uint32_t c = 0;
     int wsp = 0;
     while (mask) {
@@ -2264,7 +2269,11 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
       c = __builtin_amdgcn_readfirstlane(wnode[wv][wsp]);
       mask = wmask[wv][wsp];
     }
-    cur = kDone;
+  };
+  if constexpr (!kAny) {
+    const int g = wave_group(s, group_reach(params));
+    walk_groups(g, walk);
+    if (g >= 0) cur = kDone;
   }
   while (cur != kDone) {
     for (;;) {
@@ -2531,19 +2540,18 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
       cur = 0;
   }
   uint4 meta;
-  const uint32_t sb = __builtin_amdgcn_readfirstlane(s.sbits);
-  if (!kAny && __all(s.sbits == sb)) {
-    // Closest hit once per wavefront when the lanes' direction signs agree.
-    // A node's boxes are culled by entry alone (no distance), so the nodes a
+  auto walk = [&](uint64_t group) {
+    // Closest hit once per group of lanes that share direction signs. A node's boxes are culled by entry alone (no distance), so the nodes a
     // ray visits do not depend on its running hit, and with shared signs
     // every lane's pre-order (near child by the split axis' sign, far child
     // pushed when both boxes are entered) is one static order: the
     // wavefront walks the union of the lanes' visits in that order with one
     // stack of (node, lane mask), and each lane tests its own leaves' lines
     // in its own order, as in the per-ray loop below.
+    const uint32_t sb = __builtin_amdgcn_readlane((int)s.sbits, __builtin_ctzll(group));
     const int wv = threadIdx.x >> 6;
     const uint64_t me = 1ull << (threadIdx.x & 63u);
-    uint64_t mask = __ballot(cur == 0);
+    uint64_t mask = __ballot(cur == 0) & group;
     uint32_t c = 0;
     int wsp = 0;
     while (mask) {
@@ -2605,7 +2613,11 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
       c = __builtin_amdgcn_readfirstlane(wnode[wv][wsp]);
       mask = wmask[wv][wsp];
     }
-    cur = kDone;
+  };
+  if constexpr (!kAny) {
+    const int g = wave_group(s, group_reach(params));
+    walk_groups(g, walk);
+    if (g >= 0) cur = kDone;
   }
   while (cur != kDone) {
     for (;;) {
@@ -3053,17 +3065,17 @@ srf_status trace_sol(const Accel *a, const srf_ray *rays, uint64_t n, const floa
 srf_status trace_sph(const Accel *a, const srf_ray *rays, const srf_sphere_prev *prev,
                      uint64_t n, srf_hit *hits, hipStream_t s) {
   if (n == 0) return SRF_OK;
-  // the wavefront traversal for wavefronts of equal direction signs, then
-  // the per-lane one for the rest
+  // the wavefront traversal for groups of equal direction signs, then the
+  // per-lane one for the rest
   hipLaunchKernelGGL((k_trace_sph<false, 1>), dim3(trace_blocks(n)), dim3(kTraceBlock), 0, s,
                      (const float4 *)a->nodes, (const float4 *)a->prims, a->sorted_index, rays,
                      prev, (uint32_t)n, hits, nullptr, nullptr, max_nodes(a), (uint32_t)a->n,
-                     sph_sub(a));
+                     sph_sub(a), a->params);
   SRF_HIP(hipGetLastError());
   hipLaunchKernelGGL((k_trace_sph<false, 2>), dim3(trace_blocks(n)), dim3(kTraceBlock), 0, s,
                      (const float4 *)a->nodes, (const float4 *)a->prims, a->sorted_index, rays,
                      prev, (uint32_t)n, hits, nullptr, nullptr, max_nodes(a), (uint32_t)a->n,
-                     sph_sub(a));
+                     sph_sub(a), a->params);
   SRF_HIP(hipGetLastError());
   return SRF_OK;
 }
@@ -3103,7 +3115,8 @@ srf_status trace_any(const Accel *a, const srf_ray *rays, const float *tmax, uin
   } else
     hipLaunchKernelGGL((k_trace_sph<true, 0>), g, b, 0, s, (const float4 *)a->nodes,
                        (const float4 *)a->prims, a->sorted_index, rays, nullptr, (uint32_t)n,
-                       nullptr, tmax, occluded, max_nodes(a), (uint32_t)a->n, sph_sub(a));
+                       nullptr, tmax, occluded, max_nodes(a), (uint32_t)a->n, sph_sub(a),
+                       a->params);
   SRF_HIP(hipGetLastError());
   return SRF_OK;
 }

@@ -1,0 +1,114 @@
+"""Wavefronts whose rays do not share direction signs, on the GPU: the walks
+per group of nearby lanes and the lanes traced alone, against the oracle's
+closest hits bit for bit (triangles, tetrahedra, spheres, solids, lines) and
+its occlusion.
+
+The rays: frames seen along an axis (the signs change inside the frame) with
+sides that are no multiples of the 8x8 tile, in tile and in row order; one
+camera per ray (every lane alone); and both mixed ray by ray, so that groups
+of all sizes and lanes in no group share wavefronts.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from oracle.oracle import Oracle  # noqa: E402
+from surface_amd import workloads as W  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def S():
+    import torch
+    assert torch.cuda.is_available(), "no GPU visible"
+    from surface_amd import accel
+    return accel
+
+
+@pytest.fixture(scope="module")
+def orc():
+    return Oracle()
+
+
+# kind: geometry, the frame's eye, target and up, half extent of the scene
+def geometry(kind):
+    if kind == "tri":
+        V, F = W.heightfield(72)
+        return (V, F), ((0.5, 0.5, 2.0), (0.5, 0.5, 0.0), (0, 1, 0)), 0.5
+    if kind == "tet":
+        V, F, _ = W.tet_grid(12)
+        return (V, F), ((6.0, 6.0, 30.0), (6.0, 6.0, 6.0), (0, 1, 0)), 6.0
+    if kind == "sph":
+        P, R, _ = W.clustered_spheres(8_000, 4, 600)
+        return (P, R), ((0.0, -4.0, 0.0), (0.0, 0.0, 0.0), (0, 0, 1)), 1.0
+    if kind == "lin":
+        P, segs, _ = W.polylines(120, 40)
+        return (P, segs), ((0.0, -3.0, 0.0), (0.0, 0.0, 0.0), (0, 0, 1)), 1.0
+    V, F, _ = W.solid_grid(12, nv=int(kind[3:]))
+    return (V, F), ((6.0, 6.0, 30.0), (6.0, 6.0, 6.0), (0, 1, 0)), 6.0
+
+
+def ray_sets(view, half):
+    eye, at, up = view
+    tile = W.pinhole_rays(eye, at, up, 35.0, 101, 67)
+    row = W.pinhole_rays(eye, at, up, 35.0, 77, 45, tiled=False)
+    rng = np.random.default_rng(7)
+    n = 1500
+    single = np.zeros(n, W.RAY_DTYPE)
+    single["org"] = (np.array(at) + rng.uniform(-half, half, (n, 3))).astype(np.float32)
+    d = rng.normal(size=(n, 3))
+    single["dir"] = (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(np.float32)
+    single["flags"] = 1
+    single["prev_prim_id"] = W.NO_PRIM
+    mix = tile[:n].copy()
+    take = rng.random(n) < np.repeat(rng.uniform(0, 0.3, n // 50), 50)
+    mix[take] = single[take]
+    return {"tile": tile, "row": row, "single": single, "mix": mix}
+
+
+def build(S, orc, kind, geo):
+    A, B = geo
+    if kind == "tri":
+        a, tree = S.TriangleAccel(), orc.build_tri(A, B)
+    elif kind == "tet":
+        a, tree = S.TetraAccel(), orc.build_tet(A, B)
+    elif kind == "sph":
+        a, tree = S.ParticleAccel(), orc.build_sph(A, B)
+    elif kind == "lin":
+        a, tree = S.LineAccel(), orc.build_lin(A, B, None, 0.01)
+        a.Build(S.device_tensor(A), S.device_tensor(B), None, 0.01, True)
+        return a, lambda rays: orc.trace_lin(tree, A, B, None, 0.01, rays)
+    else:
+        nv = int(kind[3:])
+        a, tree = S.SolidAccel(), orc.build_sol(A, B, nv)
+        a.Build32(S.device_tensor(A), S.device_tensor(B), nv)
+        return a, lambda rays: orc.trace_sol(tree, A, B, rays)
+    a.Build32(S.device_tensor(A), S.device_tensor(B))
+    if kind == "sph":
+        return a, lambda rays: orc.trace_sph(tree, A, B, 0.0, rays)
+    trace = orc.trace_tri if kind == "tri" else orc.trace_tet
+    return a, lambda rays: trace(tree, A, B, rays)
+
+
+@pytest.mark.parametrize("kind", ["tri", "tet", "sph", "lin", "sol8", "sol6", "sol5"])
+def test_mixed_sign_wavefronts_match_oracle(S, orc, kind):
+    geo, view, half = geometry(kind)
+    a, oracle = build(S, orc, kind, geo)
+    for name, rays in ray_sets(view, half).items():
+        print(kind, name, len(rays), flush=True)
+        want = oracle(rays)
+        want = want[0] if isinstance(want, tuple) else want
+        dev = S.device_tensor(rays)
+        got = S.hits_to_numpy(a.Traverse(dev))
+        assert np.array_equal(got["prim_id"], want["prim_id"])
+        assert np.array_equal(got["t"].view(np.uint32), want["t"].view(np.uint32))
+        if kind != "sph":  # a sphere's u, v come from atan2 / acos
+            assert np.array_equal(got["u"], want["u"]) and np.array_equal(got["v"], want["v"])
+        hit = want["prim_id"] != W.NO_PRIM
+        assert hit.any()
+        tmax = np.where(hit, np.nextafter(want["t"], np.float32(0 if len(rays) % 2 else 1e30)),
+                        np.float32(1e30)).astype(np.float32)
+        occ = a.TraverseAny(dev, S.device_tensor(tmax)).cpu().numpy()
+        assert np.array_equal(occ != 0, hit & (want["t"] < tmax))
