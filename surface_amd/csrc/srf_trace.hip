@@ -468,6 +468,117 @@ __device__ __forceinline__ void sph_boxes(const SphSlab &r, uint32_t sb, float t
                y ? n1.x : n2.z, z ? n1.y : n2.w, l1);
 }
 
+// A leaf's spheres against the few lanes of a wavefront that visit it, as
+// (ray, sphere) pairs spread over all 64 lanes: the walks reach most leaves
+// with few lanes (3.5 of 64 in secondary trees of sorted occlusion rays, 16-30
+// for primary rays), and testing the spheres one after another leaves the
+// others idle. The rays' origins and directions wait in LDS; a pair reads its
+// ray there and its sphere with one vector load, and the pairs of a ray are
+// merged by an LDS minimum over (t, position). Used where the rounds of 64
+// pairs are at most half the spheres (a round costs about two spheres; with
+// bounds of all of them and a third, 16M spheres 2048^2 rays take 9.7 and 9.6
+// against 9.3 ms). 8M occlusion rays among 4M spheres 8.5 -> 5.4 ms, 16M
+// spheres 2048^2 rays 11.2 -> 9.3 ms, with the kernels held at 6 and 5
+// wavefronts per SIMD (5 and 4 without the bound: 5.7 and 10.6 ms).
+constexpr uint32_t kPairPrims = 16;  // spheres of a pass
+constexpr uint32_t kPairCost = 2;
+struct SphPairs {  // one wavefront's part of the block's LDS
+  float4 org[64];  // origin, previous primitive
+  float4 dir[64];  // direction, tlimit
+  unsigned long long key[64];
+  uint32_t lane[64];
+};
+__device__ __forceinline__ void sph_pairs_ray(SphPairs &P, const RaySetup &s, uint32_t prev,
+                                              float tlimit) {
+  const int l = threadIdx.x & 63;
+  P.org[l] = make_float4(s.o[0], s.o[1], s.o[2], __uint_as_float(prev));
+  P.dir[l] = make_float4(s.d[0], s.d[1], s.d[2], tlimit);
+}
+// Spheres prims[j0, j0 + count) for the lanes of `mask`. kSub: those of a big
+// leaf's secondary tree, sphere j standing at position first + sidx[j] of the
+// leaf's `nleaf`. Closest hit (no lane may have a previous primitive): a
+// sphere replaces the kept one when strictly closer, or as close, of the same
+// big leaf (`kept`) and earlier in it; equally close ones of a small leaf
+// keep the first. Returns false, with nothing changed, where a t of zero or
+// less is reported: its sign does not order as its bits do.
+template <bool kAny, bool kSub>
+__device__ __forceinline__ bool sph_pairs(SphPairs &P, uint64_t mask,
+                                          const float4 *__restrict__ prims, uint32_t j0,
+                                          uint32_t count, const uint32_t *__restrict__ sidx,
+                                          uint32_t first, uint32_t nleaf,
+                                          const uint32_t *__restrict__ sorted_index,
+                                          float &t, uint32_t &best, bool &kept, bool &occ) {
+  const uint32_t l = threadIdx.x & 63u;
+  const bool in = (mask >> l) & 1u;
+  const unsigned long long mine =
+      kAny ? 0ull : ((unsigned long long)__float_as_uint(t) << 32) | (kept ? best : 0u);
+  if (in) {
+    P.lane[__popcll(mask & ((1ull << l) - 1ull))] = l;
+    P.key[l] = mine;
+  }
+  wave_lds_sync();
+  const uint32_t pairs = __popcll(mask) * count;
+  const float rc = __builtin_amdgcn_rcpf((float)count);
+  for (uint32_t base = 0; base < pairs; base += 64) {
+    const uint32_t p = base + l;
+    bool hit = false;
+    uint32_t r = 0, q = 0;
+    float tt = 0.0f;
+    if (p < pairs) {
+      // p / count (p < 1024, count <= 16: the estimate is within 1e-4 of
+      // (p + 1/2) / count, which lies 1/32 or more from a whole number)
+      const uint32_t e = (uint32_t)(((float)p + 0.5f) * rc);
+      r = P.lane[e];
+      const uint32_t j = j0 + (p - e * count);
+      const float4 c = prims[j], a = P.org[r], b = P.dir[r];
+      RaySetup s;
+      s.o[0] = a.x;
+      s.o[1] = a.y;
+      s.o[2] = a.z;
+      s.d[0] = b.x;
+      s.d[1] = b.y;
+      s.d[2] = b.z;
+      const float zero[3] = {0.0f, 0.0f, 0.0f};
+      const float cut = kAny ? b.w : __uint_as_float((uint32_t)(P.key[r] >> 32));
+      hit = sphere_isect(s, c, INFINITY, 0.0, zero, false, cut, tt) && (!kAny || tt < b.w);
+      if (hit) {
+        q = j;
+        if (kSub) {
+          const uint32_t loc = sidx[j];
+          hit = loc < nleaf;
+          q = first + loc;
+        }
+        // an occlusion ray passes through the sphere it starts on
+        const uint32_t prev = __float_as_uint(a.w);
+        if (kAny && hit && prev != SRF_NO_PRIM) hit = sorted_index[q] != prev;
+      }
+    }
+    if (kAny) {
+      if (hit) P.key[r] = 1ull;
+    } else {
+      if (__ballot(hit && !(tt > 0.0f))) return false;
+      if (hit) atomicMin(&P.key[r], ((unsigned long long)__float_as_uint(tt) << 32) | q);
+    }
+  }
+  wave_lds_sync();
+  if (in) {
+    const unsigned long long k = P.key[l];
+    if (kAny) {
+      occ = occ || k != 0ull;
+    } else if (k < mine) {
+      t = __uint_as_float((uint32_t)(k >> 32));
+      best = (uint32_t)k;
+      kept = true;
+    }
+  }
+  wave_lds_sync();
+  return true;
+}
+// Whether `lanes` lanes and `count` spheres go as pairs.
+__device__ __forceinline__ bool sph_as_pairs(uint64_t mask, uint32_t count) {
+  return ((__popcll(mask) * count + 63u) >> 6) * kPairCost <= count;
+}
+
 // One big leaf through its secondary tree (the leaf's spheres, built as a
 // tree of their own). The reference scans the leaf in order and a sphere
 // replaces the kept one only when strictly closer, so the leaf yields the
@@ -562,9 +673,9 @@ __device__ __forceinline__ void sph_big_leaf_wave(const SphSub &sub, uint32_t nb
                                                   const uint32_t *__restrict__ sorted_index,
                                                   const RaySetup &s, uint32_t sb, uint32_t prev,
                                                   double prevT, const float prevN[3],
-                                                  float tlimit, bool in, uint32_t *wn,
-                                                  uint64_t *wm, float &t, uint32_t &best,
-                                                  bool &occ) {
+                                                  float tlimit, bool in, SphPairs &pairs,
+                                                  uint32_t *wn, uint64_t *wm, float &t,
+                                                  uint32_t &best, bool &occ) {
   const uint64_t me = 1ull << (threadIdx.x & 63u);
   const uint64_t all = __ballot(in);
   uint64_t mask = all;
@@ -620,8 +731,16 @@ __device__ __forceinline__ void sph_big_leaf_wave(const SphSub &sub, uint32_t nb
       const bool act = (mask & me) != 0;
       const uint32_t k0 = __builtin_amdgcn_readfirstlane(nd.meta.w);
       const uint32_t k1 = __builtin_amdgcn_readfirstlane(min(nd.meta.w + nd.meta.z, count));
+      const uint64_t am = __ballot(act && !(kAny && occ));
+      bool paired = false;
+      if (k1 - k0 <= kPairPrims && k0 < k1 && (kAny || !any_prev) &&
+          pbase + k1 <= sub.nprims && sph_as_pairs(am, k1 - k0) &&
+          sph_pairs<kAny, true>(pairs, am, sub.prims, pbase + k0, k1 - k0, sub.sidx, first, count,
+                                sorted_index, t, best, kept, occ)) {
+        paired = true;
+      }
       // the leaf's spheres two at a time (order and rules unchanged)
-      for (uint32_t k = k0; k < k1; k += 2) {
+      for (uint32_t k = k0; !paired && k < k1; k += 2) {
         float4 c[2];
         uint32_t loc[2];
 #pragma unroll
@@ -752,6 +871,7 @@ __device__ __forceinline__ bool sph_traverse(const float4 *__restrict__ nodes,
 // followed by part 2 on the same rays gives every ray once.
 template <bool kAny, int kPart>
 __global__ void __launch_bounds__(kTraceBlock)
+    __attribute__((amdgpu_waves_per_eu(kPart == 1 ? 5 : 1)))
 k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
             const uint32_t *__restrict__ sorted_index, const srf_ray *__restrict__ rays,
             const srf_sphere_prev *__restrict__ prevs, uint32_t n, srf_hit *__restrict__ hits,
@@ -763,8 +883,12 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   __shared__ uint32_t stack[kLanePath ? 2 * kTraceStack * kTraceBlock : 1];
   __shared__ uint32_t wnode[kWavePath ? kTraceBlock / 64 : 1][2 * kTraceStack];
   __shared__ uint64_t wmask[kWavePath ? kTraceBlock / 64 : 1][2 * kTraceStack];
-  const uint32_t i = xcd_block() * kTraceBlock + threadIdx.x;
-  if (i >= n) return;
+  __shared__ SphPairs pairs[kWavePath ? kTraceBlock / 64 : 1];
+  // the last wavefront's spare lanes trace its last ray again, unwritten: the
+  // paired leaf tests want all 64
+  const uint32_t j = xcd_block() * kTraceBlock + threadIdx.x;
+  if ((j & ~63u) >= n) return;
+  const uint32_t i = j < n ? j : n - 1;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
   double prevT = 0.0;
@@ -789,8 +913,10 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     const uint32_t sb = __builtin_amdgcn_readlane((int)s.sbits, __builtin_ctzll(mask));
     const int wv = threadIdx.x >> 6;
     const uint64_t me = 1ull << (threadIdx.x & 63u);
+    const bool prevs_any = __ballot((mask & me) != 0 && prev != SRF_NO_PRIM) != 0;
     uint32_t cur = 0;
     int wsp = 0;
+    sph_pairs_ray(pairs[wv], s, prev, FLT_MAX);
     // the descent's node in scalar registers, both children requested before
     // its boxes are tested, so the next node of the descent is in registers
     // by the time the tests have picked it
@@ -843,14 +969,20 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
           if (meta.w < nprims && meta.z <= nprims - meta.w) {
             bool unused = false;
             sph_big_leaf_wave<false>(sub, nbase, pbase, meta.w, meta.z, sorted_index, s, sb, prev,
-                                     prevT, prevN, FLT_MAX, in, &wnode[wv][kTraceStack],
-                                     &wmask[wv][kTraceStack], t, best, unused);
+                                     prevT, prevN, FLT_MAX, in, pairs[wv],
+                                     &wnode[wv][kTraceStack], &wmask[wv][kTraceStack], t, best,
+                                     unused);
           }
         } else {
           // the leaf's spheres in order, loaded two at a time
           const uint32_t q0 = __builtin_amdgcn_readfirstlane(meta.w);
           const uint32_t q1 = __builtin_amdgcn_readfirstlane(min(meta.w + meta.z, nprims));
-          for (uint32_t q = q0; q < q1; q += 2) {
+          bool kept = false, unused = false, paired = false;
+          if (q1 - q0 <= kPairPrims && q0 < q1 && !prevs_any && sph_as_pairs(mask, q1 - q0) &&
+              sph_pairs<false, false>(pairs[wv], mask, prims, q0, q1 - q0, nullptr, 0, 0,
+                                      sorted_index, t, best, kept, unused))
+            paired = true;
+          for (uint32_t q = q0; !paired && q < q1; q += 2) {
             float4 c[2];
             uint32_t sid[2];
 #pragma unroll
@@ -894,6 +1026,7 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
                                             prev, prevT, prevN, tlimit, stack + threadIdx.x, t,
                                             best);
   }
+  if (j >= n) return;
   if (kAny) {
     occluded[i] = occ ? 1u : 0u;
     return;
@@ -2745,6 +2878,7 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
 // wavefront of a plain grid. Part 1 followed by part 2 gives every ray once.
 template <int K, int kPart>
 __global__ void __launch_bounds__(kTraceBlock)
+    __attribute__((amdgpu_waves_per_eu(kPart == 1 ? 6 : 1)))
 k_any_ordered(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
               const uint32_t *__restrict__ sorted_index, const BuildParams *__restrict__ params,
               const srf_ray *__restrict__ rays, const float *__restrict__ tmax_in,
@@ -2754,6 +2888,7 @@ k_any_ordered(const float4 *__restrict__ nodes, const float4 *__restrict__ prims
   __shared__ uint32_t stack[kLanePath ? (K == kSph ? 2 : 1) * kTraceStack * kTraceBlock : 1];
   __shared__ uint32_t wnode[K == kSph && kPart != 2 ? kTraceBlock / 64 : 1][2 * kTraceStack];
   __shared__ uint64_t wmask[K == kSph && kPart != 2 ? kTraceBlock / 64 : 1][2 * kTraceStack];
+  __shared__ SphPairs pairs[K == kSph && kPart != 2 ? kTraceBlock / 64 : 1];
   uint32_t *st = stack + threadIdx.x;
   const uint32_t lane = threadIdx.x & 63u;
   uint32_t base = (counter ? blockIdx.x : xcd_block()) * kTraceBlock + (threadIdx.x & ~63u);
@@ -2764,8 +2899,10 @@ k_any_ordered(const float4 *__restrict__ nodes, const float4 *__restrict__ prims
       base = __shfl(b, 0, 64);
     }
     if (base >= n) break;
-    const uint32_t j = base + lane;
-    if (j < n) {
+    {
+      // the last group's spare lanes repeat its last ray: the paired leaf
+      // tests want all 64
+      const uint32_t j = min(base + lane, n - 1);
       const uint32_t i = order ? order[j] : j;
       uint32_t flags, prev;
       const RaySetup s = setup_ray(rays, i, flags, prev);
@@ -2810,6 +2947,7 @@ k_any_ordered(const float4 *__restrict__ nodes, const float4 *__restrict__ prims
         uint64_t mask = __ballot(1);
         uint32_t cur = 0;
         int wsp = 0;
+        sph_pairs_ray(pairs[wv], s, prev, tlimit);
         for (;;) {
           uint4 meta = make_uint4(0u, 0u, 0u, 0u);
           bool leaf = false;
@@ -2854,12 +2992,20 @@ k_any_ordered(const float4 *__restrict__ nodes, const float4 *__restrict__ prims
               const uint32_t pbase = __builtin_amdgcn_readfirstlane(__float_as_uint(nd[1].x));
               if (meta.w < nprims && meta.z <= nprims - meta.w)
                 sph_big_leaf_wave<true>(sub, nbase, pbase, meta.w, meta.z, sorted_index, s, sb,
-                                        prev, 0.0, zero, tlimit, in, &wnode[wv][kTraceStack],
-                                        &wmask[wv][kTraceStack], t, best, occ);
+                                        prev, 0.0, zero, tlimit, in, pairs[wv],
+                                        &wnode[wv][kTraceStack], &wmask[wv][kTraceStack], t,
+                                        best, occ);
             } else {
               const uint32_t q0 = __builtin_amdgcn_readfirstlane(meta.w);
               const uint32_t q1 = __builtin_amdgcn_readfirstlane(min(meta.w + meta.z, nprims));
-              for (uint32_t q = q0; q < q1; q++) {
+              const uint64_t am = __ballot(in);
+              bool kept = false;
+              const bool paired =
+                  q1 - q0 <= kPairPrims && q0 < q1 && sph_as_pairs(am, q1 - q0);
+              if (paired)
+                sph_pairs<true, false>(pairs[wv], am, prims, q0, q1 - q0, nullptr, 0, 0,
+                                       sorted_index, t, best, kept, occ);
+              for (uint32_t q = q0; !paired && q < q1; q++) {
                 const float4 c = prims[q];
                 const uint32_t sid = sorted_index[q];
                 if (!in || occ) continue;

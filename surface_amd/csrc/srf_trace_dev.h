@@ -167,6 +167,13 @@ __device__ __forceinline__ void walk_groups(int group, Walk walk) {
   }
 }
 
+// Orders a wavefront's own LDS writes before its reads (LDS operations of one
+// wavefront run in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // ---------------------------------------------------------------- triangles
 
 // TriangleIsect (Moller-Trumbore), render/render_accel_triangle.cc:1887-1938,
