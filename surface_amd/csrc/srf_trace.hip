@@ -158,6 +158,95 @@ k_trace_tri(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   }
 }
 
+// A leaf's triangles against the few lanes of a wavefront that visit it, as
+// (ray, triangle) pairs spread over all 64 lanes (sph_pairs has the same
+// form): a walk's later leaves are reached by few of its lanes -- 25 of 64 on
+// a 1024^2 frame of the 512 heightfield, 4 where a pixel tile sees many
+// triangles -- and the longest walks, which end the launch, are those with the
+// most such leaves. TestLeafNode accepts t <= the kept distance, so a leaf
+// leaves a ray its smallest t, the last triangle of equal ones: the minimum
+// over (t, ~position). Used where the rounds of 64 pairs are at most half the
+// triangles (1024^2 rays on the 512 heightfield: 732 us without pairs, 612 us
+// so; 683 and 633 us with bounds of all and a third. 333 x 251 rays on 1M
+// triangles, build included: 3270 -> 1975 us with any of the three).
+constexpr uint32_t kPairPrims = 16;  // primitives of a pass
+constexpr uint32_t kTriPairCost = 2;
+struct TriPairs {  // one wavefront's part of the block's LDS
+  float4 org[64];  // origin, previous primitive
+  float4 dir[64];  // direction, double sided
+  float4 hit[64];  // u, v, primitive
+  unsigned long long key[64];
+  uint32_t lane[64];
+};
+// Returns false, with nothing changed, where a t of zero or less or a NaN is
+// reported: its bits do not order as the values do.
+__device__ __forceinline__ bool tri_pairs(TriPairs &P, uint64_t mask,
+                                          const float4 *__restrict__ prims, uint32_t first,
+                                          uint32_t count, float kEPS, bool filter, float &t,
+                                          float &u, float &v, uint32_t &prim) {
+  const uint32_t l = threadIdx.x & 63u;
+  const bool in = (mask >> l) & 1u;
+  if (__ballot(in && !(t >= 0.0f))) return false;
+  const unsigned long long mine = ((unsigned long long)__float_as_uint(t) << 32) | 0xffffffffu;
+  if (in) {
+    P.lane[__popcll(mask & ((1ull << l) - 1ull))] = l;
+    P.key[l] = mine;
+  }
+  wave_lds_sync();
+  const uint32_t pairs = __popcll(mask) * count;
+  const float rc = __builtin_amdgcn_rcpf((float)count);
+  for (uint32_t base = 0; base < pairs; base += 64) {
+    const uint32_t p = base + l;
+    bool hit = false;
+    uint32_t r = 0;
+    float tt = 0.0f, uu = 0.0f, vv = 0.0f;
+    unsigned long long key = 0;
+    uint32_t id = 0;
+    if (p < pairs) {
+      // p / count (p < 1024, count <= 16: the estimate is within 1e-4 of
+      // (p + 1/2) / count, which lies 1/32 or more from a whole number)
+      const uint32_t e = (uint32_t)(((float)p + 0.5f) * rc);
+      const uint32_t q = first + (p - e * count);
+      const float4 *T = prims + 3 * (size_t)q;
+      const float4 A = T[0], B = T[1], C = T[2];
+      r = P.lane[e];
+      const float4 a = P.org[r], b = P.dir[r];
+      keep_loaded(A, B, C);
+      RaySetup s;
+      s.o[0] = a.x;
+      s.o[1] = a.y;
+      s.o[2] = a.z;
+      s.d[0] = b.x;
+      s.d[1] = b.y;
+      s.d[2] = b.z;
+      id = __float_as_uint(A.w);
+      hit = id != __float_as_uint(a.w) &&
+            tri_isect(s, A, B, C, b.w != 0.0f, kEPS, filter,
+                      __uint_as_float((uint32_t)(P.key[r] >> 32)), tt, uu, vv);
+      key = ((unsigned long long)__float_as_uint(tt) << 32) | (0xfffffffeu - q);
+    }
+    if (__ballot(hit)) {
+      if (__ballot(hit && !(tt > 0.0f))) return false;
+      if (hit) atomicMin(&P.key[r], key);
+      wave_lds_sync();
+      if (hit && P.key[r] == key) P.hit[r] = make_float4(uu, vv, __uint_as_float(id), 0.0f);
+      wave_lds_sync();
+    }
+  }
+  if (in) {
+    const unsigned long long k = P.key[l];
+    if (k < mine) {
+      const float4 h = P.hit[l];
+      t = __uint_as_float((uint32_t)(k >> 32));
+      u = h.x;
+      v = h.y;
+      prim = __float_as_uint(h.z);
+    }
+  }
+  wave_lds_sync();
+  return true;
+}
+
 // The wavefront traversal of k_trace_tri_wave for rays whose direction signs
 // are all SB (sign[k] << k): with the signs fixed at compile time the box
 // tests choose their near and far planes without per-lane selects.
@@ -166,8 +255,9 @@ __device__ __forceinline__ void tri_wave_closest(const float4 *__restrict__ node
                                               const float4 *__restrict__ prims,
                                               uint32_t max_nodes, uint32_t nprims,
                                               const RaySetup &s, bool ds, float kEPS,
-                                              uint32_t prev, uint32_t *wnode, uint64_t *wmask,
-                                              float &t, float &u, float &v, uint32_t &prim) {
+                                              uint32_t prev, TriPairs &pairs, uint32_t *wnode,
+                                              uint64_t *wmask, float &t, float &u, float &v,
+                                              uint32_t &prim) {
   constexpr uint32_t sb = SB;
   const bool filter = kEPS >= 1e-30f;
   const uint64_t me = 1ull << (threadIdx.x & 63u);
@@ -216,21 +306,25 @@ __device__ __forceinline__ void tri_wave_closest(const float4 *__restrict__ node
       const bool in = (mask & me) != 0;
       const uint32_t first = __builtin_amdgcn_readfirstlane(meta.w),
                      end = __builtin_amdgcn_readfirstlane(min(meta.w + meta.z, nprims));
-      for (uint32_t q = first; q < end; q += 4) {
-        // four triangles' records in one round of scalar loads (past the
+      const uint32_t cnt = end - first;
+      const bool paired = first < end && cnt <= kPairPrims &&
+                          ((__popcll(mask) * cnt + 63u) >> 6) * kTriPairCost <= cnt &&
+                          tri_pairs(pairs, mask, prims, first, cnt, kEPS, filter, t, u, v, prim);
+      for (uint32_t q = first; !paired && q < end; q += 2) {
+        // two triangles' records in one round of scalar loads (past the
         // leaf's end the last one again, unused), tested in order
-        float4 A[4], B[4], C[4];
+        float4 A[2], B[2], C[2];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < 2; j++) {
           const float4 *P = prims + 3 * (size_t)min(q + (uint32_t)j, end - 1);
           A[j] = P[0];
           B[j] = P[1];
           C[j] = P[2];
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++) keep_loaded_s(A[j], B[j], C[j]);
+        for (int j = 0; j < 2; j++) keep_loaded_s(A[j], B[j], C[j]);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < 2; j++) {
           if (q + (uint32_t)j >= end) break;
           if (in && __float_as_uint(A[j].w) != prev) {
             float tt, uu, vv;
@@ -266,38 +360,48 @@ __device__ __forceinline__ void tri_wave_closest(const float4 *__restrict__ node
 // unit). A wavefront with mixed signs runs the per-ray traversal.
 template <bool kSmall>
 __global__ void __launch_bounds__(kTraceBlock)
+    __attribute__((amdgpu_waves_per_eu(8)))
 k_trace_tri_wave(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
                  const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays,
                  uint32_t n, srf_hit *__restrict__ hits, uint32_t max_nodes, uint32_t nprims) {
-  __shared__ uint32_t stack[kSmall ? 1 : kTraceStack * kTraceBlock];
-  __shared__ uint16_t stack_lo[kSmall ? kTraceStack * kTraceBlock : 1];
-  __shared__ uint8_t stack_hi[kSmall ? kTraceStack * kTraceBlock : 1];
+  // a wavefront needs the pairs' space or its lanes' stacks, never both
+  constexpr size_t kStackBytes = kTraceStack * 64 * (kSmall ? 3 : 4);
+  constexpr size_t kBytes = kStackBytes > sizeof(TriPairs) ? kStackBytes : sizeof(TriPairs);
+  __shared__ __align__(16) unsigned char own[kTraceBlock / 64][kBytes];
   __shared__ uint32_t wnode[kTraceBlock / 64][kTraceStack];
   __shared__ uint64_t wmask[kTraceBlock / 64][kTraceStack];
-  const uint32_t i = xcd_block() * kTraceBlock + threadIdx.x;
-  if (i >= n) return;
+  // the last wavefront's spare lanes trace its last ray again, unwritten: the
+  // paired leaf tests want all 64
+  const uint32_t j = xcd_block() * kTraceBlock + threadIdx.x;
+  if ((j & ~63u) >= n) return;
+  const uint32_t i = j < n ? j : n - 1;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
   const bool ds = (flags & SRF_RAY_DOUBLE_SIDED) != 0;
   const float kEPS = FLT_EPSILON * (float)params->eps_scale;
   float t = FLT_MAX, u = 0.0f, v = 0.0f;
   uint32_t prim = SRF_NO_PRIM;
+  const uint32_t lane = threadIdx.x & 63u;
+  unsigned char *mem = own[threadIdx.x >> 6];
   const uint32_t sb = __builtin_amdgcn_readfirstlane(s.sbits);
   if (!__all(s.sbits == sb)) {
     if (kSmall)
       tri_traverse<false>(nodes, prims, max_nodes, nprims, s, ds, kEPS, prev, FLT_MAX,
-                          Stack24<kTraceBlock>{stack_lo + threadIdx.x, stack_hi + threadIdx.x},
-                          t, u, v, prim);
+                          Stack24<64>{(uint16_t *)mem + lane, mem + kTraceStack * 128 + lane}, t,
+                          u, v, prim);
     else
       tri_traverse<false>(nodes, prims, max_nodes, nprims, s, ds, kEPS, prev, FLT_MAX,
-                          Stack32<kTraceBlock>{stack + threadIdx.x}, t, u, v, prim);
+                          Stack32<64>{(uint32_t *)mem + lane}, t, u, v, prim);
   } else {
     uint32_t *wn = wnode[threadIdx.x >> 6];
     uint64_t *wm = wmask[threadIdx.x >> 6];
+    TriPairs &pairs = *reinterpret_cast<TriPairs *>(mem);
+    pairs.org[lane] = make_float4(s.o[0], s.o[1], s.o[2], __uint_as_float(prev));
+    pairs.dir[lane] = make_float4(s.d[0], s.d[1], s.d[2], ds ? 1.0f : 0.0f);
 #define SRF_TRI_WAVE(B)                                                                    \
   case B:                                                                                  \
-    tri_wave_closest<B>(nodes, prims, max_nodes, nprims, s, ds, kEPS, prev, wn, wm, t, u, v, \
-                        prim);                                                             \
+    tri_wave_closest<B>(nodes, prims, max_nodes, nprims, s, ds, kEPS, prev, pairs, wn, wm, t, \
+                        u, v, prim);                                                       \
     break;
     switch (sb) {
       SRF_TRI_WAVE(0)
@@ -314,7 +418,8 @@ k_trace_tri_wave(const float4 *__restrict__ nodes, const float4 *__restrict__ pr
 #undef SRF_TRI_WAVE
     if (prim == SRF_NO_PRIM) t = FLT_MAX;
   }
-  reinterpret_cast<float4 *>(hits)[i] = make_float4(t, u, v, __uint_as_float(prim));
+  if (j < n)
+    reinterpret_cast<float4 *>(hits)[i] = make_float4(t, u, v, __uint_as_float(prim));
 }
 
 // ------------------------------------------------------------------ spheres
@@ -480,7 +585,6 @@ __device__ __forceinline__ void sph_boxes(const SphSlab &r, uint32_t sb, float t
 // against 9.3 ms). 8M occlusion rays among 4M spheres 8.5 -> 5.4 ms, 16M
 // spheres 2048^2 rays 11.2 -> 9.3 ms, with the kernels held at 6 and 5
 // wavefronts per SIMD (5 and 4 without the bound: 5.7 and 10.6 ms).
-constexpr uint32_t kPairPrims = 16;  // spheres of a pass
 constexpr uint32_t kPairCost = 2;
 struct SphPairs {  // one wavefront's part of the block's LDS
   float4 org[64];  // origin, previous primitive
