@@ -60,22 +60,24 @@ __device__ __forceinline__ uint32_t part_by2_30(uint32_t n) {
 // on the same XCD keeps neighbouring ray tiles, which touch the same nodes or
 // voxels, on the same L2.
 constexpr uint32_t kXcds = 8;
-// Runs of SRF_XCD_GROUP consecutive blocks go to one XCD in turn: locality
-// within a run, balance across the grid (0 = one contiguous eighth per XCD,
-// 1 = the hardware's own round robin). Measured on 1024^2 ray tiles (128
-// rays per block): 128 gave the tetra trace 7.2 -> 5.4 ms and the volume
-// march 2.4 -> 2.05 ms, the triangle trace within 2 %; 0 lost 25 % on
-// triangles to imbalance between the eighths.
-#ifndef SRF_XCD_GROUP
-#define SRF_XCD_GROUP 128
-#endif
-// grids using xcd_block are padded to a multiple of this
-constexpr uint32_t kXcdPad = kXcds * (SRF_XCD_GROUP > 0 ? SRF_XCD_GROUP : 1);
-template <uint32_t kGroup = SRF_XCD_GROUP>
+// Runs of consecutive blocks go to one XCD in turn: locality within a run,
+// balance across the grid. Runs of 128 measured best on 1024^2 ray tiles (128
+// rays per block: tetra trace 7.2 -> 5.4 ms, volume march 2.4 -> 2.05 ms, the
+// triangle trace within 2 %; one contiguous eighth per XCD lost 25 % on
+// triangles to imbalance). A small grid has shorter ones, the power of two
+// that gives each XCD four or more (with runs of 128 a grid below 1024 blocks
+// left XCDs idle and one just above loads some twice: 512^2 rays through a
+// 128^3 volume, march and adjoint, 2360 -> 1741 us). The blocks after the last full set of runs keep their
+// numbers, so the renumbering is a bijection for any grid.
+constexpr uint32_t kXcdRun = 128;
 __device__ __forceinline__ uint32_t xcd_block() {
-  const uint32_t x = blockIdx.x % kXcds, k = blockIdx.x / kXcds;
-  if (kGroup == 0) return x * (gridDim.x / kXcds) + k;
-  return (k / kGroup) * (kXcds * kGroup) + x * kGroup + (k % kGroup);
+  const uint32_t per = gridDim.x / (4 * kXcds);
+  const uint32_t lg = per >= kXcdRun ? 31 - __builtin_clz(kXcdRun)
+                                     : (per ? 31 - __builtin_clz(per) : 0);
+  const uint32_t set = kXcds << lg, b = blockIdx.x;
+  if (b >= gridDim.x / set * set) return b;
+  const uint32_t x = b % kXcds, k = b / kXcds;
+  return ((k >> lg) * set) + (x << lg) + (k & ((1u << lg) - 1u));
 }
 
 // Per-build scalars produced on the device and read by later kernels.

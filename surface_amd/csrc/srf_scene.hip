@@ -787,7 +787,6 @@ srf_status scene_launch(const Scene *sc, const srf_launch_config &cfg, const srf
                      sc->depth);
   uint32_t *counter = nullptr;
   uint32_t blocks = (uint32_t)((n + block - 1) / block);
-  blocks = (blocks + kXcdPad - 1) / kXcdPad * kXcdPad;  // see xcd_block
   if (cfg.persistent) {
     const uint32_t waves = (uint32_t)((n + kChunk - 1) / kChunk);
     const uint32_t per_cu = std::max<uint32_t>(cfg.blocks_per_cu, 1u);
@@ -894,7 +893,6 @@ srf_status scene_trace_mixed(const Scene *sc, const srf_ray *rays, uint64_t n, s
       if (st != SRF_OK) return st;
     }
     uint32_t rblocks = (cn + kResolveBlock - 1) / kResolveBlock;
-    rblocks = (rblocks + kXcdPad - 1) / kXcdPad * kXcdPad;  // see xcd_block
     hipLaunchKernelGGL((k_scene_resolve<kResolveBlock>), dim3(rblocks), dim3(kResolveBlock), lds,
                        stream, sc->d_nodes, sc->num_nodes, sc->d_inst, ne, cr, cn, inv, d_off,
                        lhits, hits + c0, inst_out ? inst_out + c0 : nullptr, tdepth);

@@ -833,11 +833,8 @@ k_vol_bwd(Volume V, const float *__restrict__ tf, int N, float step,
   }
 }
 
-// blocks for n rays, padded to a multiple of kXcds (see xcd_block)
-inline uint32_t vblocks(uint64_t n, int b) {
-  const uint64_t g = (n + b - 1) / b;
-  return (uint32_t)((g + kXcdPad - 1) / kXcdPad * kXcdPad);
-}
+// blocks for n rays
+inline uint32_t vblocks(uint64_t n, int b) { return (uint32_t)((n + b - 1) / b); }
 
 }  // namespace
 }  // namespace srf
