@@ -2782,11 +2782,17 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
             srf_hit *__restrict__ hits, srf_line_hit_ext *__restrict__ ext,
             const float *__restrict__ tmax_in, uint32_t *__restrict__ occluded, uint32_t max_nodes,
             uint32_t nprims, uint32_t cap) {
-  __shared__ uint32_t st_node[kTraceStack * kTraceBlock];
+  // a wavefront needs the queue's space or its lanes' stacks, never both
+  constexpr size_t kStackBytes = kTraceStack * 64 * 4;
+  constexpr size_t kBytes = kStackBytes > sizeof(LeafQueue) ? kStackBytes : sizeof(LeafQueue);
+  __shared__ __align__(16) unsigned char own[kTraceBlock / 64][kBytes];
   __shared__ uint32_t wnode[kAny ? 1 : kTraceBlock / 64][kTraceStack];
   __shared__ uint64_t wmask[kAny ? 1 : kTraceBlock / 64][kTraceStack];
-  const uint32_t i = xcd_block() * kTraceBlock + threadIdx.x;
-  if (i >= n) return;
+  // the last wavefront's spare lanes trace its last ray again, unwritten: the
+  // queue's rounds want all 64
+  const uint32_t j = xcd_block() * kTraceBlock + threadIdx.x;
+  if ((j & ~63u) >= n) return;
+  const uint32_t i = j < n ? j : n - 1;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
   const float tlimit = kAny ? fminf(tmax_in ? tmax_in[i] : FLT_MAX, FLT_MAX) : FLT_MAX;
@@ -2794,7 +2800,8 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   uint32_t best = SRF_NO_PRIM, best_q = 0;
   bool best_cap = false;
   const BuildParams &P = *params;
-  uint32_t *sn = st_node + threadIdx.x;
+  uint32_t *sn = reinterpret_cast<uint32_t *>(own[threadIdx.x >> 6]) + (threadIdx.x & 63u);
+  LeafQueue &queue = *reinterpret_cast<LeafQueue *>(own[threadIdx.x >> 6]);
   int sp = 0;
   uint32_t cur = kDone;
   {
@@ -2805,6 +2812,19 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
       cur = 0;
   }
   uint4 meta;
+  // The line's own nearest crossing does not depend on the distance kept so
+  // far (a crossing is dropped when farther, never exchanged for another): a
+  // side replaces the kept one when not farther, a cap when strictly nearer,
+  // so of equally near crossings the last side wins, or the first cap.
+  auto test = [&](const RaySetup &r, uint32_t q, uint32_t, uint32_t &rank, float &tt) -> bool {
+    const float4 P0 = prims[2 * (size_t)q], P1 = prims[2 * (size_t)q + 1];
+    float uu, vv;
+    bool hc;
+    tt = FLT_MAX;
+    const bool hit = line_isect(tt, uu, vv, hc, P0, P1, r, cap != 0);
+    rank = hc ? kQueueSettled + 1u + rank : kQueueSettled - 1u - rank;
+    return hit;
+  };
   auto walk = [&](uint64_t group) {
     // Closest hit once per group of lanes that share direction signs. A node's boxes are culled by entry alone (no distance), so the nodes a
     // ray visits do not depend on its running hit, and with shared signs
@@ -2817,7 +2837,7 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     const int wv = threadIdx.x >> 6;
     const uint64_t me = 1ull << (threadIdx.x & 63u);
     uint64_t mask = __ballot(cur == 0) & group;
-    uint32_t c = 0;
+    uint32_t c = 0, cnt = 0;
     int wsp = 0;
     while (mask) {
       uint4 m = make_uint4(0u, 0u, 0u, 0u);
@@ -2858,31 +2878,31 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
       }
       if (leaf) {
         // TestLeafNode, render/render_accel_line.cc:579-633
-        const bool in = (mask & me) != 0;
         const uint32_t q0 = __builtin_amdgcn_readfirstlane(m.w);
         const uint32_t q1 = __builtin_amdgcn_readfirstlane(min(m.w + m.z, nprims));
-        for (uint32_t q = q0; q < q1; q++) {
-          const float4 P0 = prims[2 * (size_t)q], P1 = prims[2 * (size_t)q + 1];
-          keep_loaded_s2(P0, P1);
-          if (!in) continue;
-          bool hc;
-          if (line_isect(t, u, v, hc, P0, P1, s, cap != 0)) {
-            best = __float_as_uint(P0.w);
-            best_q = q;
-            best_cap = hc;
-          }
-        }
+        queue_leaf(queue, cnt, mask, q0, q1, test);
       }
       if (wsp == 0) break;
       --wsp;
       c = __builtin_amdgcn_readfirstlane(wnode[wv][wsp]);
       mask = wmask[wv][wsp];
     }
+    queue_run(queue, cnt, true, test);
   };
   if constexpr (!kAny) {
+    queue_start(queue, s, prev);
     const int g = wave_group(s, group_reach(params));
     walk_groups(g, walk);
-    if (g >= 0) cur = kDone;
+    if (g >= 0) {
+      cur = kDone;
+      best_q = queue.best[threadIdx.x & 63u];
+      if (best_q != SRF_NO_PRIM) {
+        const float4 P0 = prims[2 * (size_t)best_q], P1 = prims[2 * (size_t)best_q + 1];
+        line_isect(t, u, v, best_cap, P0, P1, s, cap != 0);
+        best = __float_as_uint(P0.w);
+      }
+    }
+    wave_lds_sync();
   }
   while (cur != kDone) {
     for (;;) {
@@ -2902,7 +2922,7 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
       const bool gn = nearc ? g1 : g0, gf = nearc ? g0 : g1;
       const uint32_t cn = nearc ? meta.w : meta.z, cf = nearc ? meta.z : meta.w;
       if (gn) {
-        if (gf && sp < kTraceStack) sn[(sp++) * kTraceBlock] = cf;
+        if (gf && sp < kTraceStack) sn[(sp++) * 64] = cf;
         cur = cn;
         continue;
       }
@@ -2910,7 +2930,7 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
         cur = cf;
         continue;
       }
-      cur = sp > 0 ? sn[(--sp) * kTraceBlock] : kDone;
+      cur = sp > 0 ? sn[(--sp) * 64] : kDone;
       if (cur == kDone) break;
     }
     if (cur == kDone) break;
@@ -2929,8 +2949,9 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
         best_cap = hc;
       }
     }
-    cur = sp > 0 ? sn[(--sp) * kTraceBlock] : kDone;
+    cur = sp > 0 ? sn[(--sp) * 64] : kDone;
   }
+  if (j >= n) return;
   if (kAny) {
     occluded[i] = 0u;
     return;

@@ -174,6 +174,105 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Leaf tests put off and run 64 at a time. A walk whose visits do not depend
+// on the hits found (solids and lines are never narrowed) appends a (lane,
+// primitive) entry for each test and runs them in rounds of 64, one entry a
+// lane, so that all lanes test whatever the number of lanes that reach a leaf.
+// A round's entries are in each ray's own visiting order. key[] keeps each
+// ray's best so far as (t bits, rank) with the smallest winning; rank is
+// kQueueSettled for earlier rounds' hits, so a rank below it wins ties with
+// them and one above loses.
+constexpr uint32_t kQueueLeaf = 4;  // primitives of one append
+constexpr uint32_t kQueueSettled = 0x80000000u;
+struct LeafQueue {  // one wavefront's part of the block's LDS
+  float4 org[64];   // origin, previous primitive
+  float4 dir[64];
+  unsigned long long key[64];
+  uint32_t best[64];  // primitive of key
+  uint32_t prim[64 * kQueueLeaf + 64];
+  uint8_t lane[64 * kQueueLeaf + 64];
+};
+__device__ __forceinline__ unsigned long long queue_key(float t, uint32_t rank) {
+  return ((unsigned long long)__float_as_uint(t + 0.0f) << 32) | rank;  // -0 orders as 0
+}
+__device__ __forceinline__ void queue_start(LeafQueue &Q, const RaySetup &s, uint32_t prev) {
+  const int l = threadIdx.x & 63;
+  Q.org[l] = make_float4(s.o[0], s.o[1], s.o[2], __uint_as_float(prev));
+  Q.dir[l] = make_float4(s.d[0], s.d[1], s.d[2], 0.0f);
+  Q.key[l] = queue_key(FLT_MAX, kQueueSettled);
+  Q.best[l] = SRF_NO_PRIM;
+}
+// Runs the entries in rounds of 64 (`all`: the last, partial one too) and
+// keeps the rest. test(s, prim, prev, rank, t): whether the ray s hits, at
+// which t, and its rank, given the entry's number in the round.
+template <class Test>
+__device__ __forceinline__ void queue_run(LeafQueue &Q, uint32_t &cnt, bool all, Test test) {
+  const uint32_t l = threadIdx.x & 63u;
+  uint32_t at = 0;
+  wave_lds_sync();
+  while (cnt >= at + 64u || (all && cnt > at)) {
+    bool hit = false;
+    uint32_t r = 0, q = 0;
+    unsigned long long key = 0;
+    if (at + l < cnt) {
+      q = Q.prim[at + l];
+      r = Q.lane[at + l];
+      const float4 a = Q.org[r], b = Q.dir[r];
+      RaySetup s;
+      s.o[0] = a.x;
+      s.o[1] = a.y;
+      s.o[2] = a.z;
+      s.d[0] = b.x;
+      s.d[1] = b.y;
+      s.d[2] = b.z;
+      uint32_t rank = l;
+      float t = 0.0f;
+      hit = test(s, q, __float_as_uint(a.w), rank, t);
+      key = queue_key(t, rank);
+    }
+    if (__ballot(hit)) {
+      if (hit) atomicMin(&Q.key[r], key);
+      wave_lds_sync();
+      if (hit && Q.key[r] == key) Q.best[r] = q;
+      wave_lds_sync();
+      Q.key[l] = (Q.key[l] & ~0xffffffffull) | kQueueSettled;
+    }
+    at += 64u;
+  }
+  const uint32_t rest = cnt > at ? cnt - at : 0u;
+  if (at && rest) {
+    uint32_t q = 0, r = 0;
+    if (l < rest) {
+      q = Q.prim[at + l];
+      r = Q.lane[at + l];
+    }
+    wave_lds_sync();
+    if (l < rest) {
+      Q.prim[l] = q;
+      Q.lane[l] = (uint8_t)r;
+    }
+  }
+  cnt = rest;
+}
+// Appends primitives [q0, q1) for the lanes of `mask`.
+template <class Test>
+__device__ __forceinline__ void queue_leaf(LeafQueue &Q, uint32_t &cnt, uint64_t mask, uint32_t q0,
+                                           uint32_t q1, Test test) {
+  const uint32_t l = threadIdx.x & 63u;
+  const bool in = (mask >> l) & 1u;
+  const uint32_t rank = __popcll(mask & ((1ull << l) - 1ull)), lanes = __popcll(mask);
+  for (uint32_t q = q0; q < q1; q += kQueueLeaf) {
+    const uint32_t c = min(q1 - q, kQueueLeaf);
+    if (in)
+      for (uint32_t k = 0; k < c; k++) {
+        Q.prim[cnt + rank * c + k] = q + k;
+        Q.lane[cnt + rank * c + k] = (uint8_t)l;
+      }
+    cnt += lanes * c;
+    if (cnt >= 64u) queue_run(Q, cnt, false, test);
+  }
+}
+
 // ---------------------------------------------------------------- triangles
 
 // TriangleIsect (Moller-Trumbore), render/render_accel_triangle.cc:1887-1938,
