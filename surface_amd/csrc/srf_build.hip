@@ -330,7 +330,7 @@ __device__ __forceinline__ void write_params(BuildParams *params, const Box &r) 
   p.num_nodes = 0;
   p.max_steps = 0;
   p.error = 0;
-  p.ticket = 0;
+  p.odd_box = 0;
   p.pad[0] = p.pad[1] = p.pad[2] = 0;
   *params = p;
 }
@@ -1531,6 +1531,14 @@ __device__ __forceinline__ Box merge_lr(const Box &l, const Box &r) {
 // One thread per leaf (global leaf id y): leaf box + packed primitives, the
 // leaf's own slot 0 and its parent's slot for it. With M the sorted index
 // comes from the shared scratch and is copied into the mesh's accelerator.
+// Notes a leaf box with an infinite or NaN bound (or bounds so large that
+// their sum overflows): the traversals' short box test is not for such trees.
+__device__ __forceinline__ void note_box(BuildParams *params, const Box &b) {
+  const float sum = ((fabsf(b.mn[0]) + fabsf(b.mx[0])) + (fabsf(b.mn[1]) + fabsf(b.mx[1]))) +
+                    (fabsf(b.mn[2]) + fabsf(b.mx[2]));
+  if (!(sum <= FLT_MAX)) atomicOr(&params->odd_box, 1u);
+}
+
 template <int K, bool M>
 __global__ void __launch_bounds__(256) k_leaves(uint32_t n_all, const uint32_t *sidx_all,
                                                NodeOut o, const uint32_t *total_leaves,
@@ -1560,6 +1568,7 @@ __global__ void __launch_bounds__(256) k_leaves(uint32_t n_all, const uint32_t *
   Box b;
   box_init(b);
   leaf_box_pack<K>(s, sidx, first, count, e, sg.prims, sg.sorted_faces, b);
+  note_box(params, b);
   uint32_t node = o.leaf_pos[y];
   float *words = reinterpret_cast<float *>(sg.nodes);
   {
@@ -1722,6 +1731,7 @@ __global__ void __launch_bounds__(256) k_leaves_big(const uint32_t *sidx_all, No
         b.mn[c] = mn.v;
         b.mx[c] = mx.v;
       }
+      note_box(sg.params, b);
       const uint32_t node = o.leaf_pos[y];
       float4 *w4 = reinterpret_cast<float4 *>(sg.nodes) + 4 * (size_t)node;
       w4[0] = make_float4(b.mn[0], b.mn[1], b.mn[2], 0.0f);
@@ -1858,6 +1868,7 @@ __global__ void __launch_bounds__(256) k_leaves_big_combine(const uint32_t *big,
       b.mn[c] = ex[c].v;
       b.mx[c] = ex[3 + c].v;
     }
+    note_box(sg.params, b);
     const uint32_t node = o.leaf_pos[y];
     if (node == 0 || node >= 2 * s.n - 1) {
       atomicOr(&sg.params->error, 4u);

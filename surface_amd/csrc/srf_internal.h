@@ -93,7 +93,7 @@ struct alignas(16) BuildParams {
   uint32_t num_nodes;
   uint32_t max_steps;  // deepest branch (root = 0 steps)
   uint32_t error;      // nonzero: a bounded wait gave up (never expected)
-  uint32_t ticket;     // unused (kept zero; the block keeps its 128-byte layout)
+  uint32_t odd_box;    // nonzero: some leaf's box is not finite
   uint32_t pad[3];
 };
 

@@ -248,17 +248,18 @@ __device__ __forceinline__ bool tri_pairs(TriPairs &P, uint64_t mask,
 }
 
 // The wavefront traversal of k_trace_tri_wave for rays whose direction signs
-// are all SB (sign[k] << k): with the signs fixed at compile time the box
+// are all SB (sign[k] << k; 8: those of `sbits`, for rays and trees that the
+// plain box test is not for): with the signs fixed at compile time the box
 // tests choose their near and far planes without per-lane selects.
 template <uint32_t SB>
 __device__ __forceinline__ void tri_wave_closest(const float4 *__restrict__ nodes,
                                               const float4 *__restrict__ prims,
                                               uint32_t max_nodes, uint32_t nprims,
-                                              const RaySetup &s, bool ds, float kEPS,
+                                              const RaySetup &s, uint32_t sbits, bool ds, float kEPS,
                                               uint32_t prev, TriPairs &pairs, uint32_t *wnode,
                                               uint64_t *wmask, float &t, float &u, float &v,
                                               uint32_t &prim) {
-  constexpr uint32_t sb = SB;
+  const uint32_t sb = SB < 8 ? SB : sbits;
   const bool filter = kEPS >= 1e-30f;
   const uint64_t me = 1ull << (threadIdx.x & 63u);
   uint64_t mask = __ballot(1);
@@ -279,8 +280,15 @@ __device__ __forceinline__ void tri_wave_closest(const float4 *__restrict__ node
         break;
       }
       const bool in = (mask & me) != 0;
-      const bool h0 = in && ray_aabb_wave<true>(s, SB, t, n0.x, n0.y, n0.z, n1.z, n1.w, n2.x);
-      const bool h1 = in && ray_aabb_wave<true>(s, SB, t, n0.w, n1.x, n1.y, n2.y, n2.z, n2.w);
+      bool h0, h1;
+      if (SB < 8) {
+        boxes_plain(s, SB, t, n0, n1, n2, h0, h1);
+      } else {
+        h0 = ray_aabb_wave<true>(s, sb, t, n0.x, n0.y, n0.z, n1.z, n1.w, n2.x);
+        h1 = ray_aabb_wave<true>(s, sb, t, n0.w, n1.x, n1.y, n2.y, n2.z, n2.w);
+      }
+      h0 = h0 && in;
+      h1 = h1 && in;
       const int nearc = (sb >> meta.y) & 1u;
       const uint64_t nm = __ballot(nearc ? h1 : h0), fm = __ballot(nearc ? h0 : h1);
       const uint32_t cn = nearc ? meta.w : meta.z, cf = nearc ? meta.z : meta.w;
@@ -400,10 +408,10 @@ k_trace_tri_wave(const float4 *__restrict__ nodes, const float4 *__restrict__ pr
     pairs.dir[lane] = make_float4(s.d[0], s.d[1], s.d[2], ds ? 1.0f : 0.0f);
 #define SRF_TRI_WAVE(B)                                                                    \
   case B:                                                                                  \
-    tri_wave_closest<B>(nodes, prims, max_nodes, nprims, s, ds, kEPS, prev, pairs, wn, wm, t, \
-                        u, v, prim);                                                       \
+    tri_wave_closest<B>(nodes, prims, max_nodes, nprims, s, sb, ds, kEPS, prev, pairs, wn, wm,  \
+                        t, u, v, prim);                                                    \
     break;
-    switch (sb) {
+    switch (!params->odd_box && __all(plain_ray(s)) ? sb : 8u) {
       SRF_TRI_WAVE(0)
       SRF_TRI_WAVE(1)
       SRF_TRI_WAVE(2)
@@ -412,6 +420,7 @@ k_trace_tri_wave(const float4 *__restrict__ nodes, const float4 *__restrict__ pr
       SRF_TRI_WAVE(5)
       SRF_TRI_WAVE(6)
       SRF_TRI_WAVE(7)
+      SRF_TRI_WAVE(8)
       default:
         break;
     }
@@ -2458,6 +2467,7 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     const int wv = threadIdx.x >> 6;
     const uint64_t me = 1ull << (threadIdx.x & 63u);
     uint64_t mask = __ballot(cur == 0) & group;
+    const bool plain = !params->odd_box && (__ballot(!plain_ray(s)) & group) == 0;
     uint32_t c = 0;
     int wsp = 0;
     while (mask) {
@@ -2474,11 +2484,16 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
           break;
         }
         const bool in = (mask & me) != 0;
-        float tm0, tm1;
-        const bool g0 =
-            in && box_span(s, n0.x, n0.y, n0.z, n1.z, n1.w, n2.x, tm0) && tm0 <= FLT_MAX;
-        const bool g1 =
-            in && box_span(s, n0.w, n1.x, n1.y, n2.y, n2.z, n2.w, tm1) && tm1 <= FLT_MAX;
+        bool g0, g1;
+        if (plain) {
+          boxes_plain(s, sb, FLT_MAX, n0, n1, n2, g0, g1);
+        } else {
+          float tm0, tm1;
+          g0 = box_span(s, n0.x, n0.y, n0.z, n1.z, n1.w, n2.x, tm0) && tm0 <= FLT_MAX;
+          g1 = box_span(s, n0.w, n1.x, n1.y, n2.y, n2.z, n2.w, tm1) && tm1 <= FLT_MAX;
+        }
+        g0 = g0 && in;
+        g1 = g1 && in;
         const uint32_t nearc = (sb >> m.y) & 1u;
         const uint64_t nm = __ballot(nearc ? g1 : g0), fm = __ballot(nearc ? g0 : g1);
         const uint32_t cn = nearc ? m.w : m.z, cf = nearc ? m.z : m.w;
@@ -2837,6 +2852,7 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     const int wv = threadIdx.x >> 6;
     const uint64_t me = 1ull << (threadIdx.x & 63u);
     uint64_t mask = __ballot(cur == 0) & group;
+    const bool plain = !params->odd_box && (__ballot(!plain_ray(s)) & group) == 0;
     uint32_t c = 0, cnt = 0;
     int wsp = 0;
     while (mask) {
@@ -2853,11 +2869,16 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
           break;
         }
         const bool in = (mask & me) != 0;
-        float tm0, tm1;
-        const bool g0 =
-            in && box_span(s, n0.x, n0.y, n0.z, n1.z, n1.w, n2.x, tm0) && tm0 <= FLT_MAX;
-        const bool g1 =
-            in && box_span(s, n0.w, n1.x, n1.y, n2.y, n2.z, n2.w, tm1) && tm1 <= FLT_MAX;
+        bool g0, g1;
+        if (plain) {
+          boxes_plain(s, sb, FLT_MAX, n0, n1, n2, g0, g1);
+        } else {
+          float tm0, tm1;
+          g0 = box_span(s, n0.x, n0.y, n0.z, n1.z, n1.w, n2.x, tm0) && tm0 <= FLT_MAX;
+          g1 = box_span(s, n0.w, n1.x, n1.y, n2.y, n2.z, n2.w, tm1) && tm1 <= FLT_MAX;
+        }
+        g0 = g0 && in;
+        g1 = g1 && in;
         const uint32_t nearc = (sb >> m.y) & 1u;
         const uint64_t nm = __ballot(nearc ? g1 : g0), fm = __ballot(nearc ? g0 : g1);
         const uint32_t cn = nearc ? m.w : m.z, cf = nearc ? m.z : m.w;

@@ -96,6 +96,43 @@ __device__ __forceinline__ bool ray_aabb_wave(const RaySetup &s, uint32_t sb, fl
   return (tmax > 0.0f) && (tmin <= tmax) && (tmin <= maxT);
 }
 
+// The box test where no NaN can arise: the ray's origin and the reciprocals
+// finite and not zero (plain_ray), every box finite (BuildParams::odd_box is
+// zero). Choosing the later of two entries by a comparison, as the reference
+// does, or by the hardware's maximum then gives the same values, and three
+// go in one instruction: 17 in place of 28 for a box with its planes chosen
+// (nx.. the nearer, fx.. the farther ones). The exit must lie above zero, so
+// the smallest float above zero joins the entries. Heightfield 512, 1024^2
+// rays 595 -> 555 us; 1M lines 4.93 -> 4.82 ms; solids 1 %. The sphere kernels
+// keep the comparisons: nothing gained for occlusion rays, and the closest-hit
+// kernel spills more registers (9.0 -> 9.2 ms).
+__device__ __forceinline__ bool plain_ray(const RaySetup &s) {
+  bool ok = true;
+  for (int k = 0; k < 3; k++)
+    ok = ok && fabsf(s.o[k]) <= FLT_MAX && fabsf(s.inv[k]) <= FLT_MAX && s.inv[k] != 0.0f;
+  return ok;
+}
+__device__ __forceinline__ bool box_plain(const RaySetup &s, float maxT, float nx, float ny,
+                                          float nz, float fx, float fy, float fz) {
+  const float a = (nx - s.o[0]) * s.inv[0], b = (ny - s.o[1]) * s.inv[1],
+              c = (nz - s.o[2]) * s.inv[2];
+  const float d = (fx - s.o[0]) * s.inv[0], e = (fy - s.o[1]) * s.inv[1],
+              f = (fz - s.o[2]) * s.inv[2];
+  const float enter = fmaxf(fmaxf(fmaxf(a, b), c), __uint_as_float(1u));
+  return enter <= fminf(fminf(fminf(d, e), f), maxT);
+}
+// Both boxes of a node for lanes of the signs sb (wavefront-uniform), searched
+// up to maxT.
+__device__ __forceinline__ void boxes_plain(const RaySetup &s, uint32_t sb, float maxT,
+                                            const float4 &n0, const float4 &n1, const float4 &n2,
+                                            bool &h0, bool &h1) {
+  const bool x = sb & 1u, y = sb & 2u, z = sb & 4u;
+  h0 = box_plain(s, maxT, x ? n1.z : n0.x, y ? n1.w : n0.y, z ? n2.x : n0.z, x ? n0.x : n1.z,
+                 y ? n0.y : n1.w, z ? n0.z : n2.x);
+  h1 = box_plain(s, maxT, x ? n2.y : n0.w, y ? n2.z : n1.x, z ? n2.w : n1.y, x ? n0.w : n2.y,
+                 y ? n1.x : n2.z, z ? n1.y : n2.w);
+}
+
 // ------------------------------------------------------- wavefront groups
 //
 // A wavefront traversal (one walk for many lanes, nodes and primitives loaded
