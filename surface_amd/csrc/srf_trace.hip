@@ -2104,9 +2104,14 @@ k_trace_tet(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
 // own box the ray enters is visited, nearer child first, and the closest
 // crossing wins (a solid's entry before its exit, strict <, first in visit
 // order). A crossing's point need not lie inside the solid's box (a warped
-// quad face is crossed on the plane of three of its corners), so no node or
-// solid can be skipped by distance; the kernel visits exactly the
-// reference's nodes in the reference's order.
+// quad face is crossed on the plane of three of its corners), so no node can
+// be skipped by distance; the kernel visits exactly the reference's nodes in
+// the reference's order. Its solids wait in a queue (LeafQueue) and go 64 at a
+// time through a float test that drops those missed or certainly crossed
+// beyond the kept hit (sol_may_hit), and the rest, 64 at a time, through the
+// FP64 test. 768^2 rays on 64^3 hexahedra 4.92 -> 2.76 ms (walk 0.64, filter
+// 1.6, FP64 tests 0.5; without the filter 4.39), prisms 3.06 -> 1.87, pyramids
+// 3.81 -> 2.20; 300x200 rays in row order on 40^3 hexahedra 7.7 -> 1.9 ms.
 
 // Edge i of a solid runs from vertex kSolA[i] (= i % 4 for pyramids, i % nv
 // otherwise) to kSolB[i]: GetEdges, render/render_accel_solid.cc:119-154.
@@ -2410,24 +2415,214 @@ __device__ void sol_interpolate(float d_out[8], const float p[3], const float4 *
   for (int i = NV; i < 8; i++) d_out[i] = 0.0f;
 }
 
-// Pyramids (142 VGPRs uncapped) run at 4 wavefronts per SIMD with 14 VGPRs
-// spilled (1024^2 rays on 32^3 cells of six pyramids: 8.55 -> 8.0-8.3 ms);
-// prisms and hexahedra (162 and 206 VGPRs) spill heavily under any cap and
-// are slower with one, so they are left uncapped.
+// The solid walk's queue, with the rays' frames for the filter below and the
+// entries that passed it.
+struct SolQueue {
+  LeafQueue q;
+  float4 e1[64], e2[64], dn[64];  // frame; w: |d|, coordinate bound
+  uint32_t prim2[128];
+  uint8_t lane2[128];
+};
+__device__ __forceinline__ void sol_frame(SolQueue &Q, const RaySetup &s, float cext) {
+  const int l = threadIdx.x & 63;
+  const float dd = (s.d[0] * s.d[0] + s.d[1] * s.d[1]) + s.d[2] * s.d[2];
+  const float len = __builtin_amdgcn_sqrtf(dd), il = 1.0f / len;
+  const float x = s.d[0] * il, y = s.d[1] * il, z = s.d[2] * il;
+  const bool xy = fabsf(x) > fabsf(z);
+  float ax = xy ? -y : 0.0f, ay = xy ? x : -z, az = xy ? 0.0f : y;
+  const float ia = __builtin_amdgcn_rsqf((ax * ax + ay * ay) + az * az);
+  ax *= ia;
+  ay *= ia;
+  az *= ia;
+  const float omax = fmaxf(fabsf(s.o[0]), fmaxf(fabsf(s.o[1]), fabsf(s.o[2])));
+  Q.e1[l] = make_float4(ax, ay, az, len);
+  Q.e2[l] = make_float4(y * az - z * ay, z * ax - x * az, x * ay - y * ax, cext + omax);
+  Q.dn[l] = make_float4(x, y, z, 0.0f);
+}
+
+// Whether face F's crossing certainly lies beyond the depth zt: with W the
+// weights of its corners' depths, sum (z - zt) W / sum W > 0 by more than the
+// float error (E per side product, Serr for the sum).
+template <int NV>
+__device__ __forceinline__ bool sol_beyond_of(const float *px, const float *py, const float *pz,
+                                              const float *w, const SolFace F, float zt, float E,
+                                              float Serr) {
+  auto wt = [&](int i) { return i < 0 ? -w[~i] : w[i]; };
+  float a, b, c;  // weights of corners v0, v1, v2
+  if (F.kind == 0) {
+    using Tp = SolTopo<NV>;
+    const int a2 = Tp::a(F.e2), b2 = Tp::b(F.e2), a3 = Tp::a(F.e3), b3 = Tp::b(F.e3);
+    const float x2 = px[b2] - px[a2], y2 = py[b2] - py[a2], x3 = px[b3] - px[a3],
+                y3 = py[b3] - py[a3];
+    a = wt(F.w1);
+    b = (wt(F.w2) + wt(F.w3)) + (x2 * y3 - y2 * x3);
+    c = wt(F.w0);
+  } else if (F.kind == 1) {
+    a = -wt(F.w0);
+    b = wt(F.w1);
+    c = -wt(F.w2);
+  } else {
+    a = wt(F.w0);
+    b = wt(F.w1);
+    c = wt(F.w2);
+  }
+  const float D = (a + b) + c;
+  const float S = ((pz[F.v0] - zt) * a + (pz[F.v1] - zt) * b) + (pz[F.v2] - zt) * c;
+  return (D > 20.0f * E && S > Serr) || (D < -20.0f * E && S < -Serr);
+}
+template <int NV>
+__device__ __forceinline__ bool sol_beyond(const float *px, const float *py, const float *pz,
+                                           const float *w, int f, float zt, float E, float Serr) {
+  switch (f) {
+    case 0: return sol_beyond_of<NV>(px, py, pz, w, sol_face_desc<NV>(0), zt, E, Serr);
+    case 1: return sol_beyond_of<NV>(px, py, pz, w, sol_face_desc<NV>(1), zt, E, Serr);
+    case 2: return sol_beyond_of<NV>(px, py, pz, w, sol_face_desc<NV>(2), zt, E, Serr);
+    case 3: return sol_beyond_of<NV>(px, py, pz, w, sol_face_desc<NV>(3), zt, E, Serr);
+    case 4: return sol_beyond_of<NV>(px, py, pz, w, sol_face_desc<NV>(4), zt, E, Serr);
+    default: return sol_beyond_of<NV>(px, py, pz, w, sol_face_desc<NV>(5), zt, E, Serr);
+  }
+}
+
+// False where a solid certainly has no crossing below tb: the ray misses it,
+// or crosses both faces beyond tb. The search visits every solid whose box
+// the ray enters (about 100 on the way through a 64^3 grid) and all but the
+// first few lie beyond the kept hit; this test costs a third of the FP64 one.
+//
+// Vertices are taken relative to the origin in a frame (e1, e2, d / |d|)
+// around the ray; with u = 2^-24, coordinates carry at most eta = 16 u (Z + P)
+// (differences 1u, frame 4u, dot products 3u, times sqrt 3), Z the largest
+// depth and P the largest |x| + |y|. Edge i's side product ws_i / |d| is the
+// 2D product w_i = b x a within eta (2P + 2 eta) + 4 u P^2, plus the FP64
+// side's own 1e-14 (Z + P) C (C bounds the coordinates): E. Where every |w_i|
+// exceeds E the masks, and with them the two faces, are the FP64 test's. A
+// crossing's depth is sum z W / sum W over its face's corners, W at most P^2
+// and within E (a side product), or at most 6 P^2 and within 13 E (kind 0's
+// diagonal: two side products and a product of edges, with its rounding); with
+// the sums' own rounding the W add up within 20 E, and the W (z - zt) within
+// E (32 (Z + |zt|) + 10 P). The reported t differs from depth / |d| by its
+// point's rounding to float (at most 3 ulp, kinds 1 and 2) over a component
+// above 0.1 and its own rounding, 31 u (|o| + |d| t) in all, which zt's
+// 4e-6 (C + |d| tb) covers for |d| up to 1e4.
+template <int NV>
+__device__ __forceinline__ bool sol_may_hit(const float4 *V, const RaySetup &s, const float4 &e1,
+                                            const float4 &e2, const float4 &dn, float tb) {
+  constexpr int NE = SolTopo<NV>::kEdges;
+  float px[NV], py[NV], pz[NV], w[NE];
+  float P = 0.0f, Z = 0.0f;
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    const float x = V[k].x - s.o[0], y = V[k].y - s.o[1], z = V[k].z - s.o[2];
+    px[k] = __builtin_fmaf(e1.x, x, __builtin_fmaf(e1.y, y, e1.z * z));
+    py[k] = __builtin_fmaf(e2.x, x, __builtin_fmaf(e2.y, y, e2.z * z));
+    pz[k] = __builtin_fmaf(dn.x, x, __builtin_fmaf(dn.y, y, dn.z * z));
+    P = fmaxf(P, fabsf(px[k]) + fabsf(py[k]));
+    Z = fmaxf(Z, fabsf(pz[k]));
+  }
+  const float len = e1.w, C = e2.w;
+  const float eta = 1e-6f * (Z + P);
+  const float E = (2.0f * eta * (P + eta) + 2.4e-7f * P * P) + 1e-14f * (Z + P) * C;
+  uint32_t m0 = 0;
+  float least = FLT_MAX;
+#pragma unroll
+  for (int i = 0; i < NE; i++) {
+    const int a = SolTopo<NV>::a(i), b = SolTopo<NV>::b(i);
+    w[i] = px[b] * py[a] - py[b] * px[a];
+    least = fminf(least, fabsf(w[i]));
+    m0 |= (w[i] > 0.0f ? 1u : 0u) << i;
+  }
+  const float all = ((P + Z) + fabsf(len)) + C;
+  if (!(least > E) || !(all <= FLT_MAX) || len > 1e4f) return true;
+  const uint32_t m1 = ~m0 & ((1u << NE) - 1u);
+  const int f0 = sol_face<NV>(m0, m1), f1 = sol_face<NV>(m1, m0);
+  if (f0 < 0 || f1 < 0) return false;
+  const float far = len * tb, zt = far + 4e-6f * len * (C + far);
+  const float Serr = E * (32.0f * (Z + fabsf(zt)) + 10.0f * P);
+  return !sol_beyond<NV>(px, py, pz, w, f0, zt, E, Serr) ||
+         !sol_beyond<NV>(px, py, pz, w, f1, zt, E, Serr);
+}
+
+// One solid's own nearest crossing (TestLeafNode,
+// render/render_accel_solid.cc:2206-2333): its entry, or its exit where that
+// is strictly nearer, at a distance of zero or more below `t` (kept else).
+// `ax`: the axis its distance is measured along (sol_axis).
+template <int NV>
+__device__ __forceinline__ bool sol_isect(const float4 *V, const D3 &ro, const D3 &rd,
+                                          const D3 &raypc, int ax, float &t, uint32_t &side) {
+  double ws[SolTopo<NV>::kEdges];
+  uint32_t m0, m1;
+  sol_sides<NV>(V, rd, raypc, ws, m0, m1);
+  const int f0 = sol_face<NV>(m0, m1);
+  if (f0 < 0) return false;
+  const int f1 = sol_face<NV>(m1, m0);
+  if (f1 < 0) return false;
+  const double oj = d3c(ro, ax), dj = d3c(rd, ax);
+  float c0[3], c1[3];
+  sol_point<NV>(V, ws, rd, f0, 1 << ax, c0);
+  sol_point<NV>(V, ws, rd, f1, 1 << ax, c1);
+  const float tc[2] = {(float)(((double)c0[ax] - oj) / dj), (float)(((double)c1[ax] - oj) / dj)};
+  bool hit = false;
+  for (int k = 0; k < 2; k++) {
+    if ((tc[k] >= 0.0f) && (tc[k] < t)) {
+      t = tc[k];
+      side = (uint32_t)k;
+      hit = true;
+    }
+  }
+  return hit;
+}
+// t comes from the crossing point along the last axis with |dir| > 0.1
+// (render/render_accel_solid.cc:496-500); with none (-1) the reference's t is
+// undefined and no solid is hit
+__device__ __forceinline__ int sol_axis(const RaySetup &s) {
+  int axis = -1;
+  for (int j = 0; j < 3; j++)
+    if ((double)s.d[j] > 0.1 || (double)s.d[j] < -0.1) axis = j;
+  return axis;
+}
+
+// sol_isect of the solid at P, out of line: alone it would take 224 registers
+// for hexahedra, and the walk and the filter, where the time goes, want 3
+// wavefronts per SIMD (64^3 hexahedra 3.03 -> 2.76 ms; inlined under the same
+// bound the spills land in the walk: 3.96 ms). Pyramids run at 4, where 13
+// registers spill (3: 2.28, 4: 2.20 ms).
+struct SolCross {
+  float t;
+  uint32_t side;  // 2: no crossing below the given distance
+};
+template <int NV>
+__device__ __attribute__((noinline)) SolCross sol_cross(const float4 *P, float ox, float oy,
+                                                        float oz, float dx, float dy, float dz,
+                                                        int axis) {
+  float4 V[NV];
+#pragma unroll
+  for (int k = 0; k < NV; k++) V[k] = P[k];
+  const D3 o = {ox, oy, oz}, d = {dx, dy, dz};
+  SolCross c = {FLT_MAX, 2u};
+  sol_isect<NV>(V, o, d, d3cross(d, o), axis, c.t, c.side);
+  return c;
+}
+
 template <int NV, bool kAny>
 __global__ void __launch_bounds__(kTraceBlock)
-    __attribute__((amdgpu_waves_per_eu(NV == 5 ? 4 : 1)))
+    __attribute__((amdgpu_waves_per_eu(NV == 5 ? 4 : 3)))
 k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
             const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays, uint32_t n,
             const float *__restrict__ scalars, srf_hit *__restrict__ hits,
             srf_solid_hit_ext *__restrict__ ext, const float *__restrict__ tmax_in,
             uint32_t *__restrict__ occluded, uint32_t max_nodes, uint32_t nprims) {
   constexpr int NE = SolTopo<NV>::kEdges;
-  __shared__ uint32_t st_node[kTraceStack * kTraceBlock];
+  // a wavefront needs the queue's space or its lanes' stacks, never both
+  constexpr size_t kStackBytes = kTraceStack * 64 * 4;
+  constexpr size_t kBytes =
+      kAny || kStackBytes > sizeof(SolQueue) ? kStackBytes : sizeof(SolQueue);
+  __shared__ __align__(16) unsigned char own[kTraceBlock / 64][kBytes];
   __shared__ uint32_t wnode[kAny ? 1 : kTraceBlock / 64][kTraceStack];
   __shared__ uint64_t wmask[kAny ? 1 : kTraceBlock / 64][kTraceStack];
-  const uint32_t i = xcd_block() * kTraceBlock + threadIdx.x;
-  if (i >= n) return;
+  // the last wavefront's spare lanes trace its last ray again, unwritten: the
+  // queue's rounds want all 64
+  const uint32_t ray = xcd_block() * kTraceBlock + threadIdx.x;
+  if ((ray & ~63u) >= n) return;
+  const uint32_t i = ray < n ? ray : n - 1;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
   // t_max for occlusion: the closest crossing is < t_max iff some crossing is
@@ -2436,14 +2631,11 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   uint32_t best = SRF_NO_PRIM, side = 0;
   const D3 ro = {s.o[0], s.o[1], s.o[2]}, rd = {s.d[0], s.d[1], s.d[2]};
   const D3 raypc = d3cross(rd, ro);
-  // t comes from the crossing point along the last axis with |dir| > 0.1
-  // (render/render_accel_solid.cc:496-500); with none the reference's t is
-  // undefined and no solid is hit
-  int axis = -1;
-  for (int j = 0; j < 3; j++)
-    if ((double)s.d[j] > 0.1 || (double)s.d[j] < -0.1) axis = j;
+  const int axis = sol_axis(s);
   const BuildParams &P = *params;
-  uint32_t *sn = st_node + threadIdx.x;
+  uint32_t *sn = reinterpret_cast<uint32_t *>(own[threadIdx.x >> 6]) + (threadIdx.x & 63u);
+  SolQueue &sq = *reinterpret_cast<SolQueue *>(own[threadIdx.x >> 6]);
+  LeafQueue &queue = sq.q;
   int sp = 0;
   uint32_t cur = kDone;
   {
@@ -2454,9 +2646,66 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
         tm <= FLT_MAX && axis >= 0)
       cur = 0;
   }
-  const double oj = axis == 0 ? ro.x : (axis == 1 ? ro.y : ro.z);
-  const double dj = axis == 0 ? rd.x : (axis == 1 ? rd.y : rd.z);
   uint4 meta;
+  // A solid's own nearest crossing does not depend on the distance kept so
+  // far; it replaces the kept one when strictly nearer, so of equally near
+  // ones the first wins.
+  auto test = [&](const RaySetup &r, uint32_t q, uint32_t rprev, uint32_t &rank,
+                  float &tt) -> bool {
+    const float4 *Pq = prims + (size_t)NV * q;
+    rank += kQueueSettled + 1u;
+    if (__float_as_uint(Pq[0].w) == rprev) return false;
+    const SolCross x =
+        sol_cross<NV>(Pq, r.o[0], r.o[1], r.o[2], r.d[0], r.d[1], r.d[2], sol_axis(r));
+    tt = x.t;
+    return x.side < 2u;
+  };
+  // The waiting entries 64 at a time through the filter, those that pass it
+  // 64 at a time through the test (`all`: every one).
+  auto run = [&](uint32_t &cnt, uint32_t &cnt2, bool all) {
+    const uint32_t l = threadIdx.x & 63u;
+    uint32_t at = 0;
+    wave_lds_sync();
+    while (cnt >= at + 64u || (all && cnt > at)) {
+      bool may = false;
+      uint32_t q = 0, r = 0;
+      if (at + l < cnt) {
+        q = queue.prim[at + l];
+        r = queue.lane[at + l];
+        const float4 *Pq = prims + (size_t)NV * q;
+        float4 V[NV];
+#pragma unroll
+        for (int k = 0; k < NV; k++) V[k] = Pq[k];
+        const float4 a = queue.org[r];
+        RaySetup o;
+        o.o[0] = a.x;
+        o.o[1] = a.y;
+        o.o[2] = a.z;
+        may = sol_may_hit<NV>(V, o, sq.e1[r], sq.e2[r], sq.dn[r],
+                              __uint_as_float((uint32_t)(queue.key[r] >> 32)));
+      }
+      const uint64_t m = __ballot(may);
+      if (may) {
+        const uint32_t to = cnt2 + __popcll(m & ((1ull << l) - 1ull));
+        sq.prim2[to] = q;
+        sq.lane2[to] = (uint8_t)r;
+      }
+      cnt2 += __popcll(m);
+      wave_lds_sync();
+      if (cnt2 >= 64u) {
+        queue_round(queue, sq.prim2, sq.lane2, 64u, test);
+        cnt2 = queue_keep(sq.prim2, sq.lane2, 64u, cnt2);
+        wave_lds_sync();
+      }
+      at += 64u;
+    }
+    cnt = queue_keep(queue.prim, queue.lane, at, cnt);
+    if (all && cnt2) {
+      wave_lds_sync();
+      queue_round(queue, sq.prim2, sq.lane2, cnt2, test);
+      cnt2 = 0;
+    }
+  };
   auto walk = [&](uint64_t group) {
     // Closest hit once per group of lanes that share direction signs:
     // boxes are culled by entry alone, so a ray's visits do not depend on
@@ -2468,7 +2717,7 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     const uint64_t me = 1ull << (threadIdx.x & 63u);
     uint64_t mask = __ballot(cur == 0) & group;
     const bool plain = !params->odd_box && (__ballot(!plain_ray(s)) & group) == 0;
-    uint32_t c = 0;
+    uint32_t c = 0, cnt = 0, cnt2 = 0;
     int wsp = 0;
     while (mask) {
       uint4 m = make_uint4(0u, 0u, 0u, 0u);
@@ -2512,48 +2761,32 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
           break;
         }
       }
-      if (leaf && (mask & me) != 0) {
-        // TestLeafNode, render/render_accel_solid.cc:2206-2333
+      if (leaf) {
         const uint32_t q0 = __builtin_amdgcn_readfirstlane(m.w);
         const uint32_t q1 = __builtin_amdgcn_readfirstlane(min(m.w + m.z, nprims));
-        for (uint32_t q = q0; q < q1; q++) {
-          float4 V[NV];
-          const float4 *Pq = prims + (size_t)NV * q;
-#pragma unroll
-          for (int k = 0; k < NV; k++) V[k] = Pq[k];
-          const uint32_t id = __float_as_uint(V[0].w);
-          if (id == prev) continue;
-          double ws[NE];
-          uint32_t m0, m1;
-          sol_sides<NV>(V, rd, raypc, ws, m0, m1);
-          const int f0 = sol_face<NV>(m0, m1);
-          if (f0 < 0) continue;
-          const int f1 = sol_face<NV>(m1, m0);
-          if (f1 < 0) continue;
-          float c0[3], c1[3];
-          sol_point<NV>(V, ws, rd, f0, 1 << axis, c0);
-          sol_point<NV>(V, ws, rd, f1, 1 << axis, c1);
-          const float tc[2] = {(float)(((double)c0[axis] - oj) / dj),
-                               (float)(((double)c1[axis] - oj) / dj)};
-          for (int k = 0; k < 2; k++) {
-            if ((tc[k] >= 0.0f) && (tc[k] < t)) {
-              t = tc[k];
-              best = q;
-              side = (uint32_t)k;
-            }
-          }
-        }
+        queue_leaf(queue, cnt, mask, q0, q1, [&] { run(cnt, cnt2, false); });
       }
       if (wsp == 0) break;
       --wsp;
       c = __builtin_amdgcn_readfirstlane(wnode[wv][wsp]);
       mask = wmask[wv][wsp];
     }
+    run(cnt, cnt2, true);
   };
   if constexpr (!kAny) {
+    queue_start(queue, s, prev);
+    float cext = 0.0f;
+    for (int k = 0; k < 3; k++)
+      cext = fmaxf(cext, fmaxf(fabsf(P.root_bmin[k]), fabsf(P.root_bmax[k])));
+    sol_frame(sq, s, cext);
     const int g = wave_group(s, group_reach(params));
     walk_groups(g, walk);
-    if (g >= 0) cur = kDone;
+    if (g >= 0) {
+      cur = kDone;
+      best = queue.best[threadIdx.x & 63u];
+      t = __uint_as_float((uint32_t)(queue.key[threadIdx.x & 63u] >> 32));
+    }
+    wave_lds_sync();
   }
   while (cur != kDone) {
     for (;;) {
@@ -2573,7 +2806,7 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
       const bool gn = nearc ? g1 : g0, gf = nearc ? g0 : g1;
       const uint32_t cn = nearc ? meta.w : meta.z, cf = nearc ? meta.z : meta.w;
       if (gn) {
-        if (gf && sp < kTraceStack) sn[(sp++) * kTraceBlock] = cf;
+        if (gf && sp < kTraceStack) sn[(sp++) * 64] = cf;
         cur = cn;
         continue;
       }
@@ -2581,47 +2814,29 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
         cur = cf;
         continue;
       }
-      cur = sp > 0 ? sn[(--sp) * kTraceBlock] : kDone;
+      cur = sp > 0 ? sn[(--sp) * 64] : kDone;
       if (cur == kDone) break;
     }
     if (cur == kDone) break;
     // leaf: TestLeafNode, render/render_accel_solid.cc:2206-2333
     const uint32_t count = meta.z, first = meta.w;
     for (uint32_t q = first; q < min(first + count, nprims); q++) {
-      float4 V[NV];
       const float4 *Pq = prims + (size_t)NV * q;
-#pragma unroll
-      for (int k = 0; k < NV; k++) V[k] = Pq[k];
-      const uint32_t id = __float_as_uint(V[0].w);
-      if (id == prev) continue;
-      double ws[NE];
-      uint32_t m0, m1;
-      sol_sides<NV>(V, rd, raypc, ws, m0, m1);
-      const int f0 = sol_face<NV>(m0, m1);
-      if (f0 < 0) continue;
-      const int f1 = sol_face<NV>(m1, m0);
-      if (f1 < 0) continue;
-      float c0[3], c1[3];
-      sol_point<NV>(V, ws, rd, f0, 1 << axis, c0);
-      sol_point<NV>(V, ws, rd, f1, 1 << axis, c1);
-      const float tc[2] = {(float)(((double)c0[axis] - oj) / dj),
-                           (float)(((double)c1[axis] - oj) / dj)};
-      for (int k = 0; k < 2; k++) {
-        if ((tc[k] >= 0.0f) && (tc[k] < t)) {
-          if (kAny) {
-            if (tc[k] < tlimit) {
-              occluded[i] = 1u;
-              return;
-            }
-          }
-          t = tc[k];
-          best = q;
-          side = (uint32_t)k;
+      if (__float_as_uint(Pq[0].w) == prev) continue;
+      const SolCross x = sol_cross<NV>(Pq, s.o[0], s.o[1], s.o[2], s.d[0], s.d[1], s.d[2], axis);
+      if (x.side < 2u && x.t < t) {
+        t = x.t;
+        side = x.side;
+        if (kAny && t < tlimit) {
+          occluded[i] = 1u;
+          return;
         }
+        best = q;
       }
     }
-    cur = sp > 0 ? sn[(--sp) * kTraceBlock] : kDone;
+    cur = sp > 0 ? sn[(--sp) * 64] : kDone;
   }
+  if (ray >= n) return;
   if (kAny) {
     occluded[i] = 0u;
     return;
@@ -2632,6 +2847,10 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     const float4 *Pq = prims + (size_t)NV * best;
     for (int k = 0; k < NV; k++) V[k] = Pq[k];
     prim = __float_as_uint(V[0].w);
+    // the queue keeps neither the crossing's side nor the sign of a zero
+    const SolCross x = sol_cross<NV>(Pq, s.o[0], s.o[1], s.o[2], s.d[0], s.d[1], s.d[2], axis);
+    t = x.t;
+    side = x.side & 1u;
     if (ext) {
       // the reported crossing again, in full: point, normal, weights
       double ws[NE];
@@ -2901,7 +3120,7 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
         // TestLeafNode, render/render_accel_line.cc:579-633
         const uint32_t q0 = __builtin_amdgcn_readfirstlane(m.w);
         const uint32_t q1 = __builtin_amdgcn_readfirstlane(min(m.w + m.z, nprims));
-        queue_leaf(queue, cnt, mask, q0, q1, test);
+        queue_leaf(queue, cnt, mask, q0, q1, [&] { queue_run(queue, cnt, false, test); });
       }
       if (wsp == 0) break;
       --wsp;

@@ -239,62 +239,77 @@ __device__ __forceinline__ void queue_start(LeafQueue &Q, const RaySetup &s, uin
   Q.key[l] = queue_key(FLT_MAX, kQueueSettled);
   Q.best[l] = SRF_NO_PRIM;
 }
-// Runs the entries in rounds of 64 (`all`: the last, partial one too) and
-// keeps the rest. test(s, prim, prev, rank, t): whether the ray s hits, at
-// which t, and its rank, given the entry's number in the round.
+// Runs one entry a lane: entry l of prim / lane where l < cnt. test(s, prim,
+// prev, rank, t): whether the ray s hits, at which t, and its rank, given the
+// entry's number in the round.
 template <class Test>
-__device__ __forceinline__ void queue_run(LeafQueue &Q, uint32_t &cnt, bool all, Test test) {
+__device__ __forceinline__ void queue_round(LeafQueue &Q, const uint32_t *prim,
+                                            const uint8_t *lane, uint32_t cnt, Test test) {
   const uint32_t l = threadIdx.x & 63u;
-  uint32_t at = 0;
-  wave_lds_sync();
-  while (cnt >= at + 64u || (all && cnt > at)) {
-    bool hit = false;
-    uint32_t r = 0, q = 0;
-    unsigned long long key = 0;
-    if (at + l < cnt) {
-      q = Q.prim[at + l];
-      r = Q.lane[at + l];
-      const float4 a = Q.org[r], b = Q.dir[r];
-      RaySetup s;
-      s.o[0] = a.x;
-      s.o[1] = a.y;
-      s.o[2] = a.z;
-      s.d[0] = b.x;
-      s.d[1] = b.y;
-      s.d[2] = b.z;
-      uint32_t rank = l;
-      float t = 0.0f;
-      hit = test(s, q, __float_as_uint(a.w), rank, t);
-      key = queue_key(t, rank);
-    }
-    if (__ballot(hit)) {
-      if (hit) atomicMin(&Q.key[r], key);
-      wave_lds_sync();
-      if (hit && Q.key[r] == key) Q.best[r] = q;
-      wave_lds_sync();
-      Q.key[l] = (Q.key[l] & ~0xffffffffull) | kQueueSettled;
-    }
-    at += 64u;
+  bool hit = false;
+  uint32_t r = 0, q = 0;
+  unsigned long long key = 0;
+  if (l < cnt) {
+    q = prim[l];
+    r = lane[l];
+    const float4 a = Q.org[r], b = Q.dir[r];
+    RaySetup s;
+    s.o[0] = a.x;
+    s.o[1] = a.y;
+    s.o[2] = a.z;
+    s.d[0] = b.x;
+    s.d[1] = b.y;
+    s.d[2] = b.z;
+    uint32_t rank = l;
+    float t = 0.0f;
+    hit = test(s, q, __float_as_uint(a.w), rank, t);
+    key = queue_key(t, rank);
   }
-  const uint32_t rest = cnt > at ? cnt - at : 0u;
+  if (__ballot(hit)) {
+    if (hit) atomicMin(&Q.key[r], key);
+    wave_lds_sync();
+    if (hit && Q.key[r] == key) Q.best[r] = q;
+    wave_lds_sync();
+    Q.key[l] = (Q.key[l] & ~0xffffffffull) | kQueueSettled;
+    wave_lds_sync();
+  }
+}
+// Moves entries [at, cnt) (fewer than 64 of them) to the front.
+__device__ __forceinline__ uint32_t queue_keep(uint32_t *prim, uint8_t *lane, uint32_t at,
+                                               uint32_t cnt) {
+  const uint32_t l = threadIdx.x & 63u, rest = cnt > at ? cnt - at : 0u;
   if (at && rest) {
     uint32_t q = 0, r = 0;
     if (l < rest) {
-      q = Q.prim[at + l];
-      r = Q.lane[at + l];
+      q = prim[at + l];
+      r = lane[at + l];
     }
     wave_lds_sync();
     if (l < rest) {
-      Q.prim[l] = q;
-      Q.lane[l] = (uint8_t)r;
+      prim[l] = q;
+      lane[l] = (uint8_t)r;
     }
   }
-  cnt = rest;
+  return rest;
 }
-// Appends primitives [q0, q1) for the lanes of `mask`.
+// Runs the entries in rounds of 64 (`all`: the last, partial one too) and
+// keeps the rest.
 template <class Test>
+__device__ __forceinline__ void queue_run(LeafQueue &Q, uint32_t &cnt, bool all, Test test) {
+  uint32_t at = 0;
+  wave_lds_sync();
+  while (cnt >= at + 64u || (all && cnt > at)) {
+    queue_round(Q, Q.prim + at, Q.lane + at, cnt - at, test);
+    at += 64u;
+  }
+  cnt = queue_keep(Q.prim, Q.lane, at, cnt);
+}
+
+// Appends primitives [q0, q1) for the lanes of `mask`; run() is called when
+// 64 entries or more wait.
+template <class Run>
 __device__ __forceinline__ void queue_leaf(LeafQueue &Q, uint32_t &cnt, uint64_t mask, uint32_t q0,
-                                           uint32_t q1, Test test) {
+                                           uint32_t q1, Run run) {
   const uint32_t l = threadIdx.x & 63u;
   const bool in = (mask >> l) & 1u;
   const uint32_t rank = __popcll(mask & ((1ull << l) - 1ull)), lanes = __popcll(mask);
@@ -306,7 +321,7 @@ __device__ __forceinline__ void queue_leaf(LeafQueue &Q, uint32_t &cnt, uint64_t
         Q.lane[cnt + rank * c + k] = (uint8_t)l;
       }
     cnt += lanes * c;
-    if (cnt >= 64u) queue_run(Q, cnt, false, test);
+    if (cnt >= 64u) run();
   }
 }
 
