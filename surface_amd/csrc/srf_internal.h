@@ -64,16 +64,24 @@ constexpr uint32_t kXcds = 8;
 // balance across the grid. Runs of 128 measured best on 1024^2 ray tiles (128
 // rays per block: tetra trace 7.2 -> 5.4 ms, volume march 2.4 -> 2.05 ms, the
 // triangle trace within 2 %; one contiguous eighth per XCD lost 25 % on
-// triangles to imbalance). A small grid has shorter ones, the power of two
+// triangles to imbalance). A smaller grid has shorter ones, the power of two
 // that gives each XCD four or more (with runs of 128 a grid below 1024 blocks
 // left XCDs idle and one just above loads some twice: 512^2 rays through a
-// 128^3 volume, march and adjoint, 2360 -> 1741 us). The blocks after the last full set of runs keep their
-// numbers, so the renumbering is a bijection for any grid.
-constexpr uint32_t kXcdRun = 128;
+// 128^3 volume, march and adjoint, 2360 -> 1741 us), but not below 32, a block
+// for each CU of an XCD: a handful of blocks share the loads into one L2
+// (2,013 rays on 8k triangles: 106 us on one XCD, 111 us over eight). The
+// blocks after the last full set of runs keep their numbers, so the
+// renumbering is a bijection for any grid; xcd_grid fills the smallest up to
+// one set (kernels leave blocks without work at once).
+constexpr uint32_t kXcdRunMin = 5, kXcdRunMax = 7;  // log2
+__host__ __device__ __forceinline__ uint32_t xcd_grid(uint32_t blocks) {
+  const uint32_t set = kXcds << kXcdRunMin;
+  return blocks < set ? set : blocks;
+}
 __device__ __forceinline__ uint32_t xcd_block() {
   const uint32_t per = gridDim.x / (4 * kXcds);
-  const uint32_t lg = per >= kXcdRun ? 31 - __builtin_clz(kXcdRun)
-                                     : (per ? 31 - __builtin_clz(per) : 0);
+  const uint32_t lg = per >> kXcdRunMax ? kXcdRunMax : (per >> kXcdRunMin ? 31 - __builtin_clz(per)
+                                                                        : kXcdRunMin);
   const uint32_t set = kXcds << lg, b = blockIdx.x;
   if (b >= gridDim.x / set * set) return b;
   const uint32_t x = b % kXcds, k = b / kXcds;

@@ -786,7 +786,7 @@ srf_status scene_launch(const Scene *sc, const srf_launch_config &cfg, const srf
     return set_error(SRF_ERR_UNSUPPORTED, "top-level BVH %u levels deep exceeds the LDS stack",
                      sc->depth);
   uint32_t *counter = nullptr;
-  uint32_t blocks = (uint32_t)((n + block - 1) / block);
+  uint32_t blocks = xcd_grid((uint32_t)((n + block - 1) / block));
   if (cfg.persistent) {
     const uint32_t waves = (uint32_t)((n + kChunk - 1) / kChunk);
     const uint32_t per_cu = std::max<uint32_t>(cfg.blocks_per_cu, 1u);
@@ -892,7 +892,7 @@ srf_status scene_trace_mixed(const Scene *sc, const srf_ray *rays, uint64_t n, s
                                         lhits + mx.off[e], stream);
       if (st != SRF_OK) return st;
     }
-    uint32_t rblocks = (cn + kResolveBlock - 1) / kResolveBlock;
+    const uint32_t rblocks = xcd_grid((cn + kResolveBlock - 1) / kResolveBlock);
     hipLaunchKernelGGL((k_scene_resolve<kResolveBlock>), dim3(rblocks), dim3(kResolveBlock), lds,
                        stream, sc->d_nodes, sc->num_nodes, sc->d_inst, ne, cr, cn, inv, d_off,
                        lhits, hits + c0, inst_out ? inst_out + c0 : nullptr, tdepth);

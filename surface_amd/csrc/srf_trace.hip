@@ -3509,7 +3509,7 @@ k_ao_rays_sph(const srf_ray *__restrict__ primary, const srf_hit *__restrict__ h
 
 // blocks for n rays
 inline uint32_t trace_blocks(uint64_t n) {
-  return (uint32_t)((n + kTraceBlock - 1) / kTraceBlock);
+  return xcd_grid((uint32_t)((n + kTraceBlock - 1) / kTraceBlock));
 }
 inline uint32_t max_nodes(const Accel *a) { return (uint32_t)(2 * a->n - 1); }
 // every node index fits the 3-byte stack entries

@@ -834,7 +834,7 @@ k_vol_bwd(Volume V, const float *__restrict__ tf, int N, float step,
 }
 
 // blocks for n rays
-inline uint32_t vblocks(uint64_t n, int b) { return (uint32_t)((n + b - 1) / b); }
+inline uint32_t vblocks(uint64_t n, int b) { return xcd_grid((uint32_t)((n + b - 1) / b)); }
 
 }  // namespace
 }  // namespace srf
