@@ -256,13 +256,12 @@ __device__ __forceinline__ void tri_wave_closest(const float4 *__restrict__ node
                                               const float4 *__restrict__ prims,
                                               uint32_t max_nodes, uint32_t nprims,
                                               const RaySetup &s, uint32_t sbits, bool ds, float kEPS,
-                                              uint32_t prev, TriPairs &pairs, uint32_t *wnode,
-                                              uint64_t *wmask, float &t, float &u, float &v,
-                                              uint32_t &prim) {
+                                              uint32_t prev, uint64_t mask, TriPairs &pairs,
+                                              uint32_t *wnode, uint64_t *wmask, float &t, float &u,
+                                              float &v, uint32_t &prim) {
   const uint32_t sb = SB < 8 ? SB : sbits;
   const bool filter = kEPS >= 1e-30f;
   const uint64_t me = 1ull << (threadIdx.x & 63u);
-  uint64_t mask = __ballot(1);
   uint32_t cur = 0;
   int sp = 0;
   for (;;) {
@@ -371,18 +370,17 @@ __global__ void __launch_bounds__(kTraceBlock)
     __attribute__((amdgpu_waves_per_eu(8)))
 k_trace_tri_wave(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
                  const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays,
-                 uint32_t n, srf_hit *__restrict__ hits, uint32_t max_nodes, uint32_t nprims) {
+                 uint32_t n, WaveRays lg, srf_hit *__restrict__ hits, uint32_t max_nodes,
+                 uint32_t nprims) {
   // a wavefront needs the pairs' space or its lanes' stacks, never both
   constexpr size_t kStackBytes = kTraceStack * 64 * (kSmall ? 3 : 4);
   constexpr size_t kBytes = kStackBytes > sizeof(TriPairs) ? kStackBytes : sizeof(TriPairs);
   __shared__ __align__(16) unsigned char own[kTraceBlock / 64][kBytes];
   __shared__ uint32_t wnode[kTraceBlock / 64][kTraceStack];
   __shared__ uint64_t wmask[kTraceBlock / 64][kTraceStack];
-  // the last wavefront's spare lanes trace its last ray again, unwritten: the
-  // paired leaf tests want all 64
-  const uint32_t j = xcd_block() * kTraceBlock + threadIdx.x;
-  if ((j & ~63u) >= n) return;
-  const uint32_t i = j < n ? j : n - 1;
+  WaveRay ray;
+  if (!wave_ray(rays, n, lg, ray)) return;
+  const uint32_t i = ray.i;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
   const bool ds = (flags & SRF_RAY_DOUBLE_SIDED) != 0;
@@ -393,6 +391,7 @@ k_trace_tri_wave(const float4 *__restrict__ nodes, const float4 *__restrict__ pr
   unsigned char *mem = own[threadIdx.x >> 6];
   const uint32_t sb = __builtin_amdgcn_readfirstlane(s.sbits);
   if (!__all(s.sbits == sb)) {
+    if (!ray.first) return;
     if (kSmall)
       tri_traverse<false>(nodes, prims, max_nodes, nprims, s, ds, kEPS, prev, FLT_MAX,
                           Stack24<64>{(uint16_t *)mem + lane, mem + kTraceStack * 128 + lane}, t,
@@ -408,9 +407,10 @@ k_trace_tri_wave(const float4 *__restrict__ nodes, const float4 *__restrict__ pr
     pairs.dir[lane] = make_float4(s.d[0], s.d[1], s.d[2], ds ? 1.0f : 0.0f);
 #define SRF_TRI_WAVE(B)                                                                    \
   case B:                                                                                  \
-    tri_wave_closest<B>(nodes, prims, max_nodes, nprims, s, sb, ds, kEPS, prev, pairs, wn, wm,  \
-                        t, u, v, prim);                                                    \
+    tri_wave_closest<B>(nodes, prims, max_nodes, nprims, s, sb, ds, kEPS, prev, first, pairs,   \
+                        wn, wm, t, u, v, prim);                                            \
     break;
+    const uint64_t first = __ballot(ray.first);
     switch (!params->odd_box && __all(plain_ray(s)) ? sb : 8u) {
       SRF_TRI_WAVE(0)
       SRF_TRI_WAVE(1)
@@ -427,7 +427,7 @@ k_trace_tri_wave(const float4 *__restrict__ nodes, const float4 *__restrict__ pr
 #undef SRF_TRI_WAVE
     if (prim == SRF_NO_PRIM) t = FLT_MAX;
   }
-  if (j < n)
+  if (ray.own)
     reinterpret_cast<float4 *>(hits)[i] = make_float4(t, u, v, __uint_as_float(prim));
 }
 
@@ -990,18 +990,16 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
             const srf_sphere_prev *__restrict__ prevs, uint32_t n, srf_hit *__restrict__ hits,
             const float *__restrict__ tmax_in, uint32_t *__restrict__ occluded,
             uint32_t max_nodes, uint32_t nprims, SphSub sub,
-            const BuildParams *__restrict__ params) {
+            const BuildParams *__restrict__ params, WaveRays lg) {
   constexpr bool kWavePath = !kAny && kPart != 2;
   constexpr bool kLanePath = kPart != 1;
   __shared__ uint32_t stack[kLanePath ? 2 * kTraceStack * kTraceBlock : 1];
   __shared__ uint32_t wnode[kWavePath ? kTraceBlock / 64 : 1][2 * kTraceStack];
   __shared__ uint64_t wmask[kWavePath ? kTraceBlock / 64 : 1][2 * kTraceStack];
   __shared__ SphPairs pairs[kWavePath ? kTraceBlock / 64 : 1];
-  // the last wavefront's spare lanes trace its last ray again, unwritten: the
-  // paired leaf tests want all 64
-  const uint32_t j = xcd_block() * kTraceBlock + threadIdx.x;
-  if ((j & ~63u) >= n) return;
-  const uint32_t i = j < n ? j : n - 1;
+  WaveRay ray;
+  if (!wave_ray(rays, n, lg, ray)) return;
+  const uint32_t i = ray.i;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
   double prevT = 0.0;
@@ -1128,10 +1126,10 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   };
   int group = -1;
   if constexpr (!kAny) {
-    group = wave_group(s, group_reach(params));
+    group = wave_group(s, group_reach(params), ray.first);
     if constexpr (kWavePath) walk_groups(group, walk);
     if (kPart == 1 && group < 0) return;   // left to part 2
-    if (kPart == 2 && group >= 0) return;  // done by part 1
+    if (kPart == 2 && group != -1) return;  // done by part 1
   }
   if constexpr (kLanePath) {
     if (group < 0)
@@ -1139,7 +1137,7 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
                                             prev, prevT, prevN, tlimit, stack + threadIdx.x, t,
                                             best);
   }
-  if (j >= n) return;
+  if (!ray.own) return;
   if (kAny) {
     occluded[i] = occ ? 1u : 0u;
     return;
@@ -1510,7 +1508,7 @@ template <bool kAny, bool kSmall>
 __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4)))
 k_trace_tet(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
             const uint4 *__restrict__ sorted_faces, const BuildParams *__restrict__ params,
-            const srf_ray *__restrict__ rays, uint32_t n, const float *__restrict__ scalars,
+            const srf_ray *__restrict__ rays, uint32_t n, WaveRays lg, const float *__restrict__ scalars,
             srf_hit *__restrict__ hits, srf_tet_hit_ext *__restrict__ ext,
             const float *__restrict__ tmax_in, uint32_t *__restrict__ occluded,
             uint32_t max_nodes, uint32_t nprims) {
@@ -1545,8 +1543,10 @@ k_trace_tet(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   constexpr bool kWave = kSmall && !kAny;
   __shared__ uint32_t wv_par[kSmall ? kTraceBlock / 64 : 1][kTraceStack];
   __shared__ uint64_t wv_msk[kSmall ? kTraceBlock / 64 : 1][kTraceStack];
-  const uint32_t i = xcd_block() * kTraceBlock + threadIdx.x;
-  if (i >= n) return;
+  WaveRay ray;
+  if (!wave_ray(rays, n, lg, ray)) return;
+  if (!ray.own) return;
+  const uint32_t i = ray.i;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
   const float tlimit = kAny ? (tmax_in ? tmax_in[i] : FLT_MAX) : FLT_MAX;
@@ -2606,7 +2606,7 @@ template <int NV, bool kAny>
 __global__ void __launch_bounds__(kTraceBlock)
     __attribute__((amdgpu_waves_per_eu(NV == 5 ? 4 : 3)))
 k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
-            const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays, uint32_t n,
+            const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays, uint32_t n, WaveRays lg,
             const float *__restrict__ scalars, srf_hit *__restrict__ hits,
             srf_solid_hit_ext *__restrict__ ext, const float *__restrict__ tmax_in,
             uint32_t *__restrict__ occluded, uint32_t max_nodes, uint32_t nprims) {
@@ -2618,11 +2618,9 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   __shared__ __align__(16) unsigned char own[kTraceBlock / 64][kBytes];
   __shared__ uint32_t wnode[kAny ? 1 : kTraceBlock / 64][kTraceStack];
   __shared__ uint64_t wmask[kAny ? 1 : kTraceBlock / 64][kTraceStack];
-  // the last wavefront's spare lanes trace its last ray again, unwritten: the
-  // queue's rounds want all 64
-  const uint32_t ray = xcd_block() * kTraceBlock + threadIdx.x;
-  if ((ray & ~63u) >= n) return;
-  const uint32_t i = ray < n ? ray : n - 1;
+  WaveRay ray;
+  if (!wave_ray(rays, n, lg, ray)) return;
+  const uint32_t i = ray.i;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
   // t_max for occlusion: the closest crossing is < t_max iff some crossing is
@@ -2779,10 +2777,10 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     for (int k = 0; k < 3; k++)
       cext = fmaxf(cext, fmaxf(fabsf(P.root_bmin[k]), fabsf(P.root_bmax[k])));
     sol_frame(sq, s, cext);
-    const int g = wave_group(s, group_reach(params));
+    const int g = wave_group(s, group_reach(params), ray.first);
     walk_groups(g, walk);
+    if (g != -1) cur = kDone;
     if (g >= 0) {
-      cur = kDone;
       best = queue.best[threadIdx.x & 63u];
       t = __uint_as_float((uint32_t)(queue.key[threadIdx.x & 63u] >> 32));
     }
@@ -2836,7 +2834,7 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     }
     cur = sp > 0 ? sn[(--sp) * 64] : kDone;
   }
-  if (ray >= n) return;
+  if (!ray.own) return;
   if (kAny) {
     occluded[i] = 0u;
     return;
@@ -3012,7 +3010,7 @@ __device__ __forceinline__ bool line_isect(float &t, float &u, float &v, bool &h
 template <bool kAny>
 __global__ void __launch_bounds__(kTraceBlock)
 k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
-            const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays, uint32_t n,
+            const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays, uint32_t n, WaveRays lg,
             srf_hit *__restrict__ hits, srf_line_hit_ext *__restrict__ ext,
             const float *__restrict__ tmax_in, uint32_t *__restrict__ occluded, uint32_t max_nodes,
             uint32_t nprims, uint32_t cap) {
@@ -3022,11 +3020,9 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   __shared__ __align__(16) unsigned char own[kTraceBlock / 64][kBytes];
   __shared__ uint32_t wnode[kAny ? 1 : kTraceBlock / 64][kTraceStack];
   __shared__ uint64_t wmask[kAny ? 1 : kTraceBlock / 64][kTraceStack];
-  // the last wavefront's spare lanes trace its last ray again, unwritten: the
-  // queue's rounds want all 64
-  const uint32_t j = xcd_block() * kTraceBlock + threadIdx.x;
-  if ((j & ~63u) >= n) return;
-  const uint32_t i = j < n ? j : n - 1;
+  WaveRay ray;
+  if (!wave_ray(rays, n, lg, ray)) return;
+  const uint32_t i = ray.i;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
   const float tlimit = kAny ? fminf(tmax_in ? tmax_in[i] : FLT_MAX, FLT_MAX) : FLT_MAX;
@@ -3131,10 +3127,10 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   };
   if constexpr (!kAny) {
     queue_start(queue, s, prev);
-    const int g = wave_group(s, group_reach(params));
+    const int g = wave_group(s, group_reach(params), ray.first);
     walk_groups(g, walk);
+    if (g != -1) cur = kDone;
     if (g >= 0) {
-      cur = kDone;
       best_q = queue.best[threadIdx.x & 63u];
       if (best_q != SRF_NO_PRIM) {
         const float4 P0 = prims[2 * (size_t)best_q], P1 = prims[2 * (size_t)best_q + 1];
@@ -3191,7 +3187,7 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     }
     cur = sp > 0 ? sn[(--sp) * 64] : kDone;
   }
-  if (j >= n) return;
+  if (!ray.own) return;
   if (kAny) {
     occluded[i] = 0u;
     return;
@@ -3507,9 +3503,28 @@ k_ao_rays_sph(const srf_ray *__restrict__ primary, const srf_hit *__restrict__ h
   }
 }
 
-// blocks for n rays
-inline uint32_t trace_blocks(uint64_t n) {
-  return xcd_grid((uint32_t)((n + kTraceBlock - 1) / kTraceBlock));
+// log2 of the rays a wavefront carries in a launch of n (wave_ray): the
+// fewest, 8 to 64, with which the launch has no more than `waves` wavefronts
+// (256 CUs hold 8,192 at 8 per SIMD). Measured with 64, 32, 16 and 8 (us):
+//   triangles   6k rays 380 223 174 161   83k 1470 1190 911 745
+//               262k 628 445 401 488   60k incoherent 184 162 153 171
+//   spheres     4k 1645 1140 700 506   197k 1535 1151 1213 1809
+//   hexahedra   14k 614 412 316 231   262k 1177 905 1020 1535
+//   lines       10k 763 437 284 195   77k 1015 741 681 880   320k 340 347 400 586
+// Triangle walks are the shortest, and twice the wavefronts still pay.
+// Rays that are traced one by one fill their wavefronts from 4,096 on.
+constexpr uint64_t kTriWaves = 16384, kWaves = 8192, kAloneWaves = 4096;
+constexpr WaveRays kFullWaves = {6u, 6u};
+inline WaveRays wave_rays(uint64_t n, uint64_t waves) {
+  WaveRays w = {3u, 3u};
+  while (w.lg < 6 && (n >> w.lg) > waves) w.lg++;
+  while (w.lg_alone < 6 && (n >> w.lg_alone) > kAloneWaves) w.lg_alone++;
+  if (w.lg_alone < w.lg) w.lg_alone = w.lg;
+  return w;
+}
+// blocks for n rays, carried as w says
+inline uint32_t trace_blocks(uint64_t n, WaveRays w = kFullWaves) {
+  return xcd_grid(wave_run_blocks(n, w) << (w.lg_alone - w.lg));
 }
 inline uint32_t max_nodes(const Accel *a) { return (uint32_t)(2 * a->n - 1); }
 // every node index fits the 3-byte stack entries
@@ -3533,14 +3548,15 @@ inline SphSub sph_sub(const Accel *a) {
 srf_status trace_tri(const Accel *a, const srf_ray *rays, uint64_t n, srf_hit *hits,
                      hipStream_t s) {
   if (n == 0) return SRF_OK;
+  const WaveRays lg = wave_rays(n, kTriWaves);
   if (small_nodes(a))
-    hipLaunchKernelGGL((k_trace_tri_wave<true>), dim3(trace_blocks(n)), dim3(kTraceBlock), 0, s,
+    hipLaunchKernelGGL((k_trace_tri_wave<true>), dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0, s,
                        (const float4 *)a->nodes, (const float4 *)a->prims, a->params, rays,
-                       (uint32_t)n, hits, max_nodes(a), (uint32_t)a->n);
+                       (uint32_t)n, lg, hits, max_nodes(a), (uint32_t)a->n);
   else
-    hipLaunchKernelGGL((k_trace_tri_wave<false>), dim3(trace_blocks(n)), dim3(kTraceBlock), 0,
+    hipLaunchKernelGGL((k_trace_tri_wave<false>), dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0,
                        s, (const float4 *)a->nodes, (const float4 *)a->prims, a->params, rays,
-                       (uint32_t)n, hits, max_nodes(a), (uint32_t)a->n);
+                       (uint32_t)n, lg, hits, max_nodes(a), (uint32_t)a->n);
   SRF_HIP(hipGetLastError());
   return SRF_OK;
 }
@@ -3548,15 +3564,18 @@ srf_status trace_tri(const Accel *a, const srf_ray *rays, uint64_t n, srf_hit *h
 srf_status trace_tet(const Accel *a, const srf_ray *rays, uint64_t n, const float *scalars,
                      srf_hit *hits, srf_tet_hit_ext *ext, hipStream_t s) {
   if (n == 0) return SRF_OK;
+  const WaveRays lg = wave_rays(n, kWaves);
   if (small_tet(a))
-    hipLaunchKernelGGL((k_trace_tet<false, true>), dim3(trace_blocks(n)), dim3(kTraceBlock), 0,
+    hipLaunchKernelGGL((k_trace_tet<false, true>), dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0,
                        s, (const float4 *)a->nodes, (const float4 *)a->prims,
-                       (const uint4 *)a->sorted_faces, a->params, rays, (uint32_t)n, scalars,
+                       (const uint4 *)a->sorted_faces, a->params, rays, (uint32_t)n, lg,
+                       scalars,
                        hits, ext, nullptr, nullptr, max_nodes(a), (uint32_t)a->n);
   else
-    hipLaunchKernelGGL((k_trace_tet<false, false>), dim3(trace_blocks(n)), dim3(kTraceBlock), 0,
+    hipLaunchKernelGGL((k_trace_tet<false, false>), dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0,
                        s, (const float4 *)a->nodes, (const float4 *)a->prims,
-                       (const uint4 *)a->sorted_faces, a->params, rays, (uint32_t)n, scalars,
+                       (const uint4 *)a->sorted_faces, a->params, rays, (uint32_t)n, lg,
+                       scalars,
                        hits, ext, nullptr, nullptr, max_nodes(a), (uint32_t)a->n);
   SRF_HIP(hipGetLastError());
   return SRF_OK;
@@ -3566,16 +3585,17 @@ template <bool kAny>
 srf_status launch_sol(const Accel *a, const srf_ray *rays, uint64_t n, const float *scalars,
                       srf_hit *hits, srf_solid_hit_ext *ext, const float *tmax,
                       uint32_t *occluded, hipStream_t s) {
-  const dim3 g(trace_blocks(n)), b(kTraceBlock);
+  const WaveRays lg = kAny ? kFullWaves : wave_rays(n, kWaves);
+  const dim3 g(trace_blocks(n, lg)), b(kTraceBlock);
   const float4 *nd = (const float4 *)a->nodes, *pr = (const float4 *)a->prims;
   if (a->nvps == 5)
-    hipLaunchKernelGGL((k_trace_sol<5, kAny>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n,
+    hipLaunchKernelGGL((k_trace_sol<5, kAny>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n, lg,
                        scalars, hits, ext, tmax, occluded, max_nodes(a), (uint32_t)a->n);
   else if (a->nvps == 6)
-    hipLaunchKernelGGL((k_trace_sol<6, kAny>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n,
+    hipLaunchKernelGGL((k_trace_sol<6, kAny>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n, lg,
                        scalars, hits, ext, tmax, occluded, max_nodes(a), (uint32_t)a->n);
   else if (a->nvps == 8)
-    hipLaunchKernelGGL((k_trace_sol<8, kAny>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n,
+    hipLaunchKernelGGL((k_trace_sol<8, kAny>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n, lg,
                        scalars, hits, ext, tmax, occluded, max_nodes(a), (uint32_t)a->n);
   else
     return set_error(SRF_ERR_INTERNAL, "solid accelerator with %u vertices per solid", a->nvps);
@@ -3586,9 +3606,10 @@ srf_status launch_sol(const Accel *a, const srf_ray *rays, uint64_t n, const flo
 srf_status trace_lin(const Accel *a, const srf_ray *rays, uint64_t n, srf_hit *hits,
                      srf_line_hit_ext *ext, hipStream_t s) {
   if (n == 0) return SRF_OK;
-  hipLaunchKernelGGL(k_trace_lin<false>, dim3(trace_blocks(n)), dim3(kTraceBlock), 0, s,
+  const WaveRays lg = wave_rays(n, kWaves);
+  hipLaunchKernelGGL(k_trace_lin<false>, dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0, s,
                      (const float4 *)a->nodes, (const float4 *)a->prims, a->params, rays,
-                     (uint32_t)n, hits, ext, nullptr, nullptr, max_nodes(a), (uint32_t)a->n,
+                     (uint32_t)n, lg, hits, ext, nullptr, nullptr, max_nodes(a), (uint32_t)a->n,
                      a->line_cap);
   SRF_HIP(hipGetLastError());
   return SRF_OK;
@@ -3603,17 +3624,18 @@ srf_status trace_sol(const Accel *a, const srf_ray *rays, uint64_t n, const floa
 srf_status trace_sph(const Accel *a, const srf_ray *rays, const srf_sphere_prev *prev,
                      uint64_t n, srf_hit *hits, hipStream_t s) {
   if (n == 0) return SRF_OK;
+  const WaveRays lg = wave_rays(n, kWaves);
   // the wavefront traversal for groups of equal direction signs, then the
   // per-lane one for the rest
-  hipLaunchKernelGGL((k_trace_sph<false, 1>), dim3(trace_blocks(n)), dim3(kTraceBlock), 0, s,
+  hipLaunchKernelGGL((k_trace_sph<false, 1>), dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0, s,
                      (const float4 *)a->nodes, (const float4 *)a->prims, a->sorted_index, rays,
                      prev, (uint32_t)n, hits, nullptr, nullptr, max_nodes(a), (uint32_t)a->n,
-                     sph_sub(a), a->params);
+                     sph_sub(a), a->params, lg);
   SRF_HIP(hipGetLastError());
-  hipLaunchKernelGGL((k_trace_sph<false, 2>), dim3(trace_blocks(n)), dim3(kTraceBlock), 0, s,
+  hipLaunchKernelGGL((k_trace_sph<false, 2>), dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0, s,
                      (const float4 *)a->nodes, (const float4 *)a->prims, a->sorted_index, rays,
                      prev, (uint32_t)n, hits, nullptr, nullptr, max_nodes(a), (uint32_t)a->n,
-                     sph_sub(a), a->params);
+                     sph_sub(a), a->params, lg);
   SRF_HIP(hipGetLastError());
   return SRF_OK;
 }
@@ -3625,7 +3647,7 @@ srf_status trace_any(const Accel *a, const srf_ray *rays, const float *tmax, uin
   if (a->kind == kLin) {
     hipLaunchKernelGGL(k_trace_lin<true>, dim3(trace_blocks(n)), dim3(kTraceBlock), 0, s,
                        (const float4 *)a->nodes, (const float4 *)a->prims, a->params, rays,
-                       (uint32_t)n, nullptr, nullptr, tmax, occluded, max_nodes(a),
+                       (uint32_t)n, kFullWaves, nullptr, nullptr, tmax, occluded, max_nodes(a),
                        (uint32_t)a->n, a->line_cap);
     SRF_HIP(hipGetLastError());
     return SRF_OK;
@@ -3643,18 +3665,18 @@ srf_status trace_any(const Accel *a, const srf_ray *rays, const float *tmax, uin
     if (small_tet(a))
       hipLaunchKernelGGL((k_trace_tet<true, true>), g, b, 0, s, (const float4 *)a->nodes,
                          (const float4 *)a->prims, (const uint4 *)a->sorted_faces, a->params,
-                         rays, (uint32_t)n, nullptr, nullptr, nullptr, tmax, occluded,
+                         rays, (uint32_t)n, kFullWaves, nullptr, nullptr, nullptr, tmax, occluded,
                          max_nodes(a), (uint32_t)a->n);
     else
       hipLaunchKernelGGL((k_trace_tet<true, false>), g, b, 0, s, (const float4 *)a->nodes,
                          (const float4 *)a->prims, (const uint4 *)a->sorted_faces, a->params,
-                         rays, (uint32_t)n, nullptr, nullptr, nullptr, tmax, occluded,
+                         rays, (uint32_t)n, kFullWaves, nullptr, nullptr, nullptr, tmax, occluded,
                          max_nodes(a), (uint32_t)a->n);
   } else
     hipLaunchKernelGGL((k_trace_sph<true, 0>), g, b, 0, s, (const float4 *)a->nodes,
                        (const float4 *)a->prims, a->sorted_index, rays, nullptr, (uint32_t)n,
                        nullptr, tmax, occluded, max_nodes(a), (uint32_t)a->n, sph_sub(a),
-                       a->params);
+                       a->params, kFullWaves);
   SRF_HIP(hipGetLastError());
   return SRF_OK;
 }

@@ -133,6 +133,74 @@ __device__ __forceinline__ void boxes_plain(const RaySetup &s, uint32_t sb, floa
                  y ? n1.x : n2.z, z ? n1.y : n2.w);
 }
 
+// ---------------------------------------------------- rays of a wavefront
+//
+// A wavefront carries 2^lg rays: 64 where a launch has enough of them to fill
+// the chip, fewer below that (wave_rays). Fewer rays share a shorter walk, so
+// a small launch, which is as long as its longest wavefronts, ends sooner; its
+// idle lanes cost nothing and take part in paired and queued tests. Rays that
+// will mostly be traced one by one, a lane each, want their wavefronts full
+// at smaller launches: where fewer than half of the 2^lg parts of a run of
+// 2^lg_alone rays share direction signs, the run stays in one wavefront, and
+// those of its other parts leave (250k random rays on 8k triangles: 158 us in
+// wavefronts of 64, 310 us in 16s). The grid holds the first parts of all runs,
+// then the second ones and so on: blocks that leave are together at its end
+// (with a run's parts in neighbouring blocks the ones that stay fall on every
+// fourth CU: 450 us).
+struct WaveRays {
+  uint32_t lg, lg_alone;  // lg <= lg_alone
+};
+// blocks that one part of every run takes
+__host__ __device__ __forceinline__ uint32_t wave_run_blocks(uint64_t n, WaveRays w) {
+  const uint32_t lg = w.lg_alone + 31 - __builtin_clz(kTraceBlock / 64);
+  return (uint32_t)((n + (1ull << lg) - 1) >> lg);
+}
+struct WaveRay {
+  uint32_t i;  // this lane's ray
+  bool first;  // the lane stands for its ray (the others repeat one)
+  bool own;    // and writes its result
+};
+// False for a wavefront without rays. The lanes beyond the wavefront's rays,
+// and the last one's beyond n, repeat a ray: the paired and queued leaf tests
+// want all 64 lanes.
+__device__ __forceinline__ bool wave_ray(const srf_ray *__restrict__ rays, uint32_t n, WaveRays w,
+                                         WaveRay &r) {
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t lg = w.lg;
+  uint32_t block = xcd_block(), part_no = 0;
+  const uint32_t lg_parts = w.lg_alone - lg;
+  const uint32_t run_blocks = wave_run_blocks(n, w);
+  for (; part_no < (1u << lg_parts) && block >= run_blocks; part_no++) block -= run_blocks;
+  if (part_no >> lg_parts) return false;
+  const uint64_t from = (uint64_t)__builtin_amdgcn_readfirstlane(
+                            block * (kTraceBlock / 64) + (threadIdx.x >> 6))
+                        << w.lg_alone;
+  const uint64_t base = from + ((uint64_t)part_no << lg);
+  if (base >= n) return false;
+  if (lg_parts) {
+    const uint32_t run = 1u << w.lg_alone, part = 1u << lg;
+    const uint64_t k = from + (lane & (run - 1u));
+    const float *d = rays[k < n ? k : n - 1].dir;
+    const uint64_t x = __ballot(d[0] < 0.0f), y = __ballot(d[1] < 0.0f), z = __ballot(d[2] < 0.0f);
+    uint32_t same = 0;
+    for (uint32_t at = 0; at < run; at += part) {
+      const uint64_t m = (part == 64u ? ~0ull : (1ull << part) - 1ull) << at;
+      same += ((x & m) == 0 || (x & m) == m) && ((y & m) == 0 || (y & m) == m) &&
+              ((z & m) == 0 || (z & m) == m);
+    }
+    if (2 * same < run / part) {
+      if (base != from) return false;
+      lg = w.lg_alone;
+    }
+  }
+  const uint32_t count = 1u << lg;
+  const uint32_t j = (uint32_t)base + (lane & (count - 1u));
+  r.i = j < n ? j : n - 1;
+  r.first = lane < count;
+  r.own = r.first && j < n;
+  return true;
+}
+
 // ------------------------------------------------------- wavefront groups
 //
 // A wavefront traversal (one walk for many lanes, nodes and primitives loaded
@@ -174,14 +242,14 @@ __device__ __forceinline__ uint64_t next_group(const RaySetup &s, uint64_t todo,
   return (__ballot(same) & todo) | (1ull << lead);
 }
 
-// The number of this lane's group, -1 for a lane that is traced alone. Lanes
-// of one sign are group 0. Up to kGroupTries groups are kept whatever their
+// The number of this lane's group, -1 for a lane that is traced alone, -2 for
+// one that repeats another's ray (`first` false). Lanes of one sign are group 0. Up to kGroupTries groups are kept whatever their
 // sizes; where the lanes do not fit in so many, only groups of kGroupMin
 // lanes or more.
-__device__ __forceinline__ int wave_group(const RaySetup &s, float reach) {
+__device__ __forceinline__ int wave_group(const RaySetup &s, float reach, bool first) {
   const uint32_t sb = __builtin_amdgcn_readfirstlane(s.sbits);
-  if (__all(s.sbits == sb)) return 0;
-  uint64_t todo = __ballot(1);
+  if (__all(s.sbits == sb)) return first ? 0 : -2;
+  uint64_t todo = __ballot(first);
   const int lane = threadIdx.x & 63;
   int group = -1, size = 0;
   for (int g = 0; g < kGroupTries && todo; g++) {
@@ -192,6 +260,7 @@ __device__ __forceinline__ int wave_group(const RaySetup &s, float reach) {
       size = __popcll(m);
     }
   }
+  if (!first) return -2;
   return todo && size < kGroupMin ? -1 : group;
 }
 
