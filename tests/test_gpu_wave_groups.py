@@ -112,3 +112,32 @@ def test_mixed_sign_wavefronts_match_oracle(S, orc, kind):
                         np.float32(1e30)).astype(np.float32)
         occ = a.TraverseAny(dev, S.device_tensor(tmax)).cpu().numpy()
         assert np.array_equal(occ != 0, hit & (want["t"] < tmax))
+
+
+# launches that carry 8, 16, 32 and 64 rays per wavefront, coherent and not
+# (random rays of one wavefront stay together from 262,144 / 64 runs on), at
+# sizes around a run of 64 and a block
+@pytest.mark.parametrize("kind", ["tri", "sph", "lin", "tet", "sol8"])
+@pytest.mark.parametrize("n", [1, 63, 65, 127, 129, 40_007, 150_001, 280_000])
+def test_launch_sizes_match_oracle(S, orc, kind, n):
+    geo, (eye, at, up), half = geometry(kind)
+    a, oracle = build(S, orc, kind, geo)
+    side = int(np.ceil(np.sqrt(n)))
+    frame = W.pinhole_rays(eye, at, up, 35.0, side, side)[:n]
+    rng = np.random.default_rng(n)
+    rand = frame.copy()
+    rand["org"] = (np.array(at) + rng.uniform(-half, half, (n, 3))).astype(np.float32)
+    d = rng.normal(size=(n, 3))
+    rand["dir"] = (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(np.float32)
+    half_rand = frame.copy()
+    mix = (np.arange(n) // 64) % 3 == 1
+    half_rand[mix] = rand[mix]
+    check = np.arange(n) if n < 1000 else np.unique(np.r_[0:200, n - 200:n,
+                                                          rng.integers(0, n, 4000)])
+    for rays in (frame, rand, half_rand):
+        got = S.hits_to_numpy(a.Traverse(S.device_tensor(rays)))
+        assert len(got) == n
+        want = oracle(np.ascontiguousarray(rays[check]))
+        want = want[0] if isinstance(want, tuple) else want
+        assert np.array_equal(got["prim_id"][check], want["prim_id"])
+        assert np.array_equal(got["t"][check].view(np.uint32), want["t"].view(np.uint32))
