@@ -86,12 +86,13 @@ REF_COUNTS = {
 OWN_LOADS = {"k_trace_tet": (0.9458 + 0.0588, 0.4413 + 0.0187)}
 # HBM bytes per launch (FETCH_SIZE x 2 + WRITE_SIZE, KiB -> bytes) from the
 # counter passes over `bench.py --probe` summarised in
-# profiles/counters_bench_probe.md; a configuration missing here reports null
+# profiles/counters_bench_probe.md and, for the triangle and sphere kernels,
+# profiles/counters_full_lanes.md; a configuration missing here reports null
 TRAFFIC = {
-    "heightfield512": 212_830_143,
-    "heightfield725": 452_779_556,
+    "heightfield512": 174_836_000,
+    "heightfield725": 359_670_000,
     "tetgrid64": 131_817_300,
-    "plummer16M_primary": 1_425_300_605,  # both launches
+    "plummer16M_primary": 1_176_510_000,  # both launches
     "scene64_upper": 23_603_015_759,      # persistent launch, 128-lane blocks
     "k_vol_fwd": 275_953_791,             # the march without checkpoints
     "k_vol_bwd": 1_376_455_261,
