@@ -613,7 +613,8 @@ __device__ __forceinline__ void sph_pairs_ray(SphPairs &P, const RaySetup &s, ui
 // sphere replaces the kept one when strictly closer, or as close, of the same
 // big leaf (`kept`) and earlier in it; equally close ones of a small leaf
 // keep the first. Returns false, with nothing changed, where a t of zero or
-// less is reported: its sign does not order as its bits do.
+// less is reported: its sign does not order as its bits do. A kept t of -0 (a
+// ray that starts on a sphere, tangent to it) enters the keys as +0.
 template <bool kAny, bool kSub>
 __device__ __forceinline__ bool sph_pairs(SphPairs &P, uint64_t mask,
                                           const float4 *__restrict__ prims, uint32_t j0,
@@ -624,7 +625,8 @@ __device__ __forceinline__ bool sph_pairs(SphPairs &P, uint64_t mask,
   const uint32_t l = threadIdx.x & 63u;
   const bool in = (mask >> l) & 1u;
   const unsigned long long mine =
-      kAny ? 0ull : ((unsigned long long)__float_as_uint(t) << 32) | (kept ? best : 0u);
+      kAny ? 0ull
+           : ((unsigned long long)__float_as_uint(t + 0.0f) << 32) | (kept ? best : 0u);
   if (in) {
     P.lane[__popcll(mask & ((1ull << l) - 1ull))] = l;
     P.key[l] = mine;
