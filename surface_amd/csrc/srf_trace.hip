@@ -2604,22 +2604,25 @@ __device__ __attribute__((noinline)) SolCross sol_cross(const float4 *P, float o
   return c;
 }
 
-template <int NV, bool kAny>
+// kPart: 0 occlusion, a lane a ray; closest hits in two launches, 1 the lanes
+// in groups that share direction signs, 2 the lanes in no group, a lane a ray.
+// A lane's own walk has the FP64 test inline, without a register cap (pyramids
+// at 4 wavefronts per SIMD, 14 VGPRs spilled): with the call at every solid it
+// is 1.3 to 2.7 times as slow.
+template <int NV, int kPart>
 __global__ void __launch_bounds__(kTraceBlock)
-    __attribute__((amdgpu_waves_per_eu(NV == 5 ? 4 : 3)))
+    __attribute__((amdgpu_waves_per_eu(NV == 5 ? 4 : kPart == 1 ? 3 : 1)))
 k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
-            const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays, uint32_t n, WaveRays lg,
-            const float *__restrict__ scalars, srf_hit *__restrict__ hits,
+            const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays, uint32_t n,
+            WaveRays lg, const float *__restrict__ scalars, srf_hit *__restrict__ hits,
             srf_solid_hit_ext *__restrict__ ext, const float *__restrict__ tmax_in,
             uint32_t *__restrict__ occluded, uint32_t max_nodes, uint32_t nprims) {
+  constexpr bool kAny = kPart == 0, kWave = kPart == 1;
   constexpr int NE = SolTopo<NV>::kEdges;
-  // a wavefront needs the queue's space or its lanes' stacks, never both
-  constexpr size_t kStackBytes = kTraceStack * 64 * 4;
-  constexpr size_t kBytes =
-      kAny || kStackBytes > sizeof(SolQueue) ? kStackBytes : sizeof(SolQueue);
-  __shared__ __align__(16) unsigned char own[kTraceBlock / 64][kBytes];
-  __shared__ uint32_t wnode[kAny ? 1 : kTraceBlock / 64][kTraceStack];
-  __shared__ uint64_t wmask[kAny ? 1 : kTraceBlock / 64][kTraceStack];
+  __shared__ uint32_t st_node[kWave ? 1 : kTraceStack * kTraceBlock];
+  __shared__ SolQueue queues[kWave ? kTraceBlock / 64 : 1];
+  __shared__ uint32_t wnode[kWave ? kTraceBlock / 64 : 1][kTraceStack];
+  __shared__ uint64_t wmask[kWave ? kTraceBlock / 64 : 1][kTraceStack];
   WaveRay ray;
   if (!wave_ray(rays, n, lg, ray)) return;
   const uint32_t i = ray.i;
@@ -2633,8 +2636,8 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   const D3 raypc = d3cross(rd, ro);
   const int axis = sol_axis(s);
   const BuildParams &P = *params;
-  uint32_t *sn = reinterpret_cast<uint32_t *>(own[threadIdx.x >> 6]) + (threadIdx.x & 63u);
-  SolQueue &sq = *reinterpret_cast<SolQueue *>(own[threadIdx.x >> 6]);
+  uint32_t *sn = st_node + threadIdx.x;
+  SolQueue &sq = queues[kWave ? threadIdx.x >> 6 : 0];
   LeafQueue &queue = sq.q;
   int sp = 0;
   uint32_t cur = kDone;
@@ -2773,22 +2776,21 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     }
     run(cnt, cnt2, true);
   };
-  if constexpr (!kAny) {
+  int group = -1;
+  if constexpr (!kAny) group = wave_group(s, group_reach(params), ray.first);
+  if constexpr (kWave) {
     queue_start(queue, s, prev);
     float cext = 0.0f;
     for (int k = 0; k < 3; k++)
       cext = fmaxf(cext, fmaxf(fabsf(P.root_bmin[k]), fabsf(P.root_bmax[k])));
     sol_frame(sq, s, cext);
-    const int g = wave_group(s, group_reach(params), ray.first);
-    walk_groups(g, walk);
-    if (g != -1) cur = kDone;
-    if (g >= 0) {
-      best = queue.best[threadIdx.x & 63u];
-      t = __uint_as_float((uint32_t)(queue.key[threadIdx.x & 63u] >> 32));
-    }
-    wave_lds_sync();
+    walk_groups(group, walk);
+    if (group < 0) return;  // left to part 2
+    best = queue.best[threadIdx.x & 63u];
+    cur = kDone;
   }
-  while (cur != kDone) {
+  if (kPart == 2 && group != -1) return;  // done by part 1
+  while (!kWave && cur != kDone) {
     for (;;) {
       if (cur >= max_nodes) {
         cur = kDone;
@@ -2806,7 +2808,7 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
       const bool gn = nearc ? g1 : g0, gf = nearc ? g0 : g1;
       const uint32_t cn = nearc ? meta.w : meta.z, cf = nearc ? meta.z : meta.w;
       if (gn) {
-        if (gf && sp < kTraceStack) sn[(sp++) * 64] = cf;
+        if (gf && sp < kTraceStack) sn[(sp++) * kTraceBlock] = cf;
         cur = cn;
         continue;
       }
@@ -2814,19 +2816,19 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
         cur = cf;
         continue;
       }
-      cur = sp > 0 ? sn[(--sp) * 64] : kDone;
+      cur = sp > 0 ? sn[(--sp) * kTraceBlock] : kDone;
       if (cur == kDone) break;
     }
     if (cur == kDone) break;
     // leaf: TestLeafNode, render/render_accel_solid.cc:2206-2333
     const uint32_t count = meta.z, first = meta.w;
     for (uint32_t q = first; q < min(first + count, nprims); q++) {
+      float4 V[NV];
       const float4 *Pq = prims + (size_t)NV * q;
-      if (__float_as_uint(Pq[0].w) == prev) continue;
-      const SolCross x = sol_cross<NV>(Pq, s.o[0], s.o[1], s.o[2], s.d[0], s.d[1], s.d[2], axis);
-      if (x.side < 2u && x.t < t) {
-        t = x.t;
-        side = x.side;
+#pragma unroll
+      for (int k = 0; k < NV; k++) V[k] = Pq[k];
+      if (__float_as_uint(V[0].w) == prev) continue;
+      if (sol_isect<NV>(V, ro, rd, raypc, axis, t, side)) {
         if (kAny && t < tlimit) {
           occluded[i] = 1u;
           return;
@@ -2834,7 +2836,7 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
         best = q;
       }
     }
-    cur = sp > 0 ? sn[(--sp) * 64] : kDone;
+    cur = sp > 0 ? sn[(--sp) * kTraceBlock] : kDone;
   }
   if (!ray.own) return;
   if (kAny) {
@@ -2847,10 +2849,11 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     const float4 *Pq = prims + (size_t)NV * best;
     for (int k = 0; k < NV; k++) V[k] = Pq[k];
     prim = __float_as_uint(V[0].w);
-    // the queue keeps neither the crossing's side nor the sign of a zero
-    const SolCross x = sol_cross<NV>(Pq, s.o[0], s.o[1], s.o[2], s.d[0], s.d[1], s.d[2], axis);
-    t = x.t;
-    side = x.side & 1u;
+    if (kWave) {  // the queue keeps neither the crossing's side nor the sign of a zero
+      const SolCross x = sol_cross<NV>(Pq, s.o[0], s.o[1], s.o[2], s.d[0], s.d[1], s.d[2], axis);
+      t = x.t;
+      side = x.side & 1u;
+    }
     if (ext) {
       // the reported crossing again, in full: point, normal, weights
       double ws[NE];
@@ -3583,22 +3586,21 @@ srf_status trace_tet(const Accel *a, const srf_ray *rays, uint64_t n, const floa
   return SRF_OK;
 }
 
-template <bool kAny>
-srf_status launch_sol(const Accel *a, const srf_ray *rays, uint64_t n, const float *scalars,
-                      srf_hit *hits, srf_solid_hit_ext *ext, const float *tmax,
-                      uint32_t *occluded, hipStream_t s) {
-  const WaveRays lg = kAny ? kFullWaves : wave_rays(n, kWaves);
+template <int kPart>
+srf_status launch_sol(const Accel *a, const srf_ray *rays, uint64_t n, WaveRays lg,
+                      const float *scalars, srf_hit *hits, srf_solid_hit_ext *ext,
+                      const float *tmax, uint32_t *occluded, hipStream_t s) {
   const dim3 g(trace_blocks(n, lg)), b(kTraceBlock);
   const float4 *nd = (const float4 *)a->nodes, *pr = (const float4 *)a->prims;
   if (a->nvps == 5)
-    hipLaunchKernelGGL((k_trace_sol<5, kAny>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n, lg,
-                       scalars, hits, ext, tmax, occluded, max_nodes(a), (uint32_t)a->n);
+    hipLaunchKernelGGL((k_trace_sol<5, kPart>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n,
+                       lg, scalars, hits, ext, tmax, occluded, max_nodes(a), (uint32_t)a->n);
   else if (a->nvps == 6)
-    hipLaunchKernelGGL((k_trace_sol<6, kAny>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n, lg,
-                       scalars, hits, ext, tmax, occluded, max_nodes(a), (uint32_t)a->n);
+    hipLaunchKernelGGL((k_trace_sol<6, kPart>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n,
+                       lg, scalars, hits, ext, tmax, occluded, max_nodes(a), (uint32_t)a->n);
   else if (a->nvps == 8)
-    hipLaunchKernelGGL((k_trace_sol<8, kAny>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n, lg,
-                       scalars, hits, ext, tmax, occluded, max_nodes(a), (uint32_t)a->n);
+    hipLaunchKernelGGL((k_trace_sol<8, kPart>), g, b, 0, s, nd, pr, a->params, rays, (uint32_t)n,
+                       lg, scalars, hits, ext, tmax, occluded, max_nodes(a), (uint32_t)a->n);
   else
     return set_error(SRF_ERR_INTERNAL, "solid accelerator with %u vertices per solid", a->nvps);
   SRF_HIP(hipGetLastError());
@@ -3620,7 +3622,10 @@ srf_status trace_lin(const Accel *a, const srf_ray *rays, uint64_t n, srf_hit *h
 srf_status trace_sol(const Accel *a, const srf_ray *rays, uint64_t n, const float *scalars,
                      srf_hit *hits, srf_solid_hit_ext *ext, hipStream_t s) {
   if (n == 0) return SRF_OK;
-  return launch_sol<false>(a, rays, n, scalars, hits, ext, nullptr, nullptr, s);
+  const WaveRays lg = wave_rays(n, kWaves);
+  const srf_status st = launch_sol<1>(a, rays, n, lg, scalars, hits, ext, nullptr, nullptr, s);
+  if (st != SRF_OK) return st;
+  return launch_sol<2>(a, rays, n, lg, scalars, hits, ext, nullptr, nullptr, s);
 }
 
 srf_status trace_sph(const Accel *a, const srf_ray *rays, const srf_sphere_prev *prev,
@@ -3645,7 +3650,8 @@ srf_status trace_sph(const Accel *a, const srf_ray *rays, const srf_sphere_prev 
 srf_status trace_any(const Accel *a, const srf_ray *rays, const float *tmax, uint64_t n,
                      uint32_t *occluded, hipStream_t s) {
   if (n == 0) return SRF_OK;
-  if (a->kind == kSol) return launch_sol<true>(a, rays, n, nullptr, nullptr, nullptr, tmax, occluded, s);
+  if (a->kind == kSol)
+    return launch_sol<0>(a, rays, n, kFullWaves, nullptr, nullptr, nullptr, tmax, occluded, s);
   if (a->kind == kLin) {
     hipLaunchKernelGGL(k_trace_lin<true>, dim3(trace_blocks(n)), dim3(kTraceBlock), 0, s,
                        (const float4 *)a->nodes, (const float4 *)a->prims, a->params, rays,
