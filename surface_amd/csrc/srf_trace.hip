@@ -978,12 +978,12 @@ __device__ __forceinline__ bool sph_traverse(const float4 *__restrict__ nodes,
   return false;
 }
 
-// Closest hit (and plain occlusion) of spheres. kPart selects the lanes a
+// Closest hit (and plain occlusion) of spheres. kPart selects the rays a
 // launch handles: 0 all, 1 the groups that share direction signs
 // (walk_groups: the wavefront traversal; no per-lane stack, so the launch
-// holds more wavefronts per CU), 2 the lanes in no group (the per-lane
-// traversal). Part 1
-// followed by part 2 on the same rays gives every ray once.
+// holds more wavefronts per CU), 2 the rays that part 1 marked (leave_alone),
+// a lane a ray. Part 1 followed by part 2 on the same rays gives every
+// ray once.
 template <bool kAny, int kPart>
 __global__ void __launch_bounds__(kTraceBlock)
     __attribute__((amdgpu_waves_per_eu(kPart == 1 ? 5 : 1)))
@@ -993,14 +993,13 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
             const float *__restrict__ tmax_in, uint32_t *__restrict__ occluded,
             uint32_t max_nodes, uint32_t nprims, SphSub sub,
             const BuildParams *__restrict__ params, WaveRays lg) {
-  constexpr bool kWavePath = !kAny && kPart != 2;
-  constexpr bool kLanePath = kPart != 1;
-  __shared__ uint32_t stack[kLanePath ? 2 * kTraceStack * kTraceBlock : 1];
+  constexpr bool kWavePath = kPart == 1;
+  __shared__ uint32_t stack[kWavePath ? 1 : 2 * kTraceStack * kTraceBlock];
   __shared__ uint32_t wnode[kWavePath ? kTraceBlock / 64 : 1][2 * kTraceStack];
   __shared__ uint64_t wmask[kWavePath ? kTraceBlock / 64 : 1][2 * kTraceStack];
   __shared__ SphPairs pairs[kWavePath ? kTraceBlock / 64 : 1];
   WaveRay ray;
-  if (!wave_ray(rays, n, lg, ray)) return;
+  if (kPart == 2 ? !ray_alone(hits, n, lg.lg, ray) : !wave_ray(rays, n, lg, ray)) return;
   const uint32_t i = ray.i;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
@@ -1126,18 +1125,15 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
       have = false;
     }
   };
-  int group = -1;
-  if constexpr (!kAny) {
-    group = wave_group(s, group_reach(params), ray.first);
-    if constexpr (kWavePath) walk_groups(group, walk);
-    if (kPart == 1 && group < 0) return;   // left to part 2
-    if (kPart == 2 && group != -1) return;  // done by part 1
-  }
-  if constexpr (kLanePath) {
-    if (group < 0)
-      occ = sph_traverse<kAny, kTraceBlock>(nodes, prims, sorted_index, max_nodes, nprims, sub, s,
-                                            prev, prevT, prevN, tlimit, stack + threadIdx.x, t,
-                                            best);
+  if constexpr (kWavePath) {
+    const int group = wave_group(s, group_reach(params), ray.first);
+    walk_groups(group, walk);
+    if (group == -1) leave_alone(hits, ray);
+    if (group < 0) return;
+  } else {
+    occ = sph_traverse<kAny, kTraceBlock>(nodes, prims, sorted_index, max_nodes, nprims, sub, s,
+                                          prev, prevT, prevN, tlimit, stack + threadIdx.x, t,
+                                          best);
   }
   if (!ray.own) return;
   if (kAny) {
@@ -2604,9 +2600,9 @@ __device__ __attribute__((noinline)) SolCross sol_cross(const float4 *P, float o
   return c;
 }
 
-// kPart: 0 occlusion, a lane a ray; closest hits in two launches, 1 the lanes
-// in groups that share direction signs, 2 the lanes in no group, a lane a ray.
-// A lane's own walk has the FP64 test inline, without a register cap (pyramids
+// kPart: 0 occlusion, a lane a ray; closest hits in two launches, 1 the groups
+// that share direction signs, 2 the rays that part 1 marked (leave_alone), a
+// lane a ray in full wavefronts. A lane's own walk has the FP64 test inline, without a register cap (pyramids
 // at 4 wavefronts per SIMD, 14 VGPRs spilled): with the call at every solid it
 // is 1.3 to 2.7 times as slow.
 template <int NV, int kPart>
@@ -2624,7 +2620,7 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   __shared__ uint32_t wnode[kWave ? kTraceBlock / 64 : 1][kTraceStack];
   __shared__ uint64_t wmask[kWave ? kTraceBlock / 64 : 1][kTraceStack];
   WaveRay ray;
-  if (!wave_ray(rays, n, lg, ray)) return;
+  if (kPart == 2 ? !ray_alone(hits, n, lg.lg, ray) : !wave_ray(rays, n, lg, ray)) return;
   const uint32_t i = ray.i;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
@@ -2776,20 +2772,22 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     }
     run(cnt, cnt2, true);
   };
-  int group = -1;
-  if constexpr (!kAny) group = wave_group(s, group_reach(params), ray.first);
   if constexpr (kWave) {
     queue_start(queue, s, prev);
     float cext = 0.0f;
     for (int k = 0; k < 3; k++)
       cext = fmaxf(cext, fmaxf(fabsf(P.root_bmin[k]), fabsf(P.root_bmax[k])));
     sol_frame(sq, s, cext);
+    const int group = wave_group(s, group_reach(params), ray.first);
     walk_groups(group, walk);
-    if (group < 0) return;  // left to part 2
+    if (group == -1) leave_alone(hits, ray);
+    if (group < 0) return;
     best = queue.best[threadIdx.x & 63u];
     cur = kDone;
   }
-  if (kPart == 2 && group != -1) return;  // done by part 1
+  // a lane a ray: sol_isect spelled out (3-6 % faster than the call inlined)
+  const double oj = axis == 0 ? ro.x : (axis == 1 ? ro.y : ro.z);
+  const double dj = axis == 0 ? rd.x : (axis == 1 ? rd.y : rd.z);
   while (!kWave && cur != kDone) {
     for (;;) {
       if (cur >= max_nodes) {
@@ -2828,12 +2826,30 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
 #pragma unroll
       for (int k = 0; k < NV; k++) V[k] = Pq[k];
       if (__float_as_uint(V[0].w) == prev) continue;
-      if (sol_isect<NV>(V, ro, rd, raypc, axis, t, side)) {
-        if (kAny && t < tlimit) {
-          occluded[i] = 1u;
-          return;
+      double ws[NE];
+      uint32_t m0, m1;
+      sol_sides<NV>(V, rd, raypc, ws, m0, m1);
+      const int f0 = sol_face<NV>(m0, m1);
+      if (f0 < 0) continue;
+      const int f1 = sol_face<NV>(m1, m0);
+      if (f1 < 0) continue;
+      float c0[3], c1[3];
+      sol_point<NV>(V, ws, rd, f0, 1 << axis, c0);
+      sol_point<NV>(V, ws, rd, f1, 1 << axis, c1);
+      const float tc[2] = {(float)(((double)c0[axis] - oj) / dj),
+                           (float)(((double)c1[axis] - oj) / dj)};
+      for (int k = 0; k < 2; k++) {
+        if ((tc[k] >= 0.0f) && (tc[k] < t)) {
+          if (kAny) {
+            if (tc[k] < tlimit) {
+              occluded[i] = 1u;
+              return;
+            }
+          }
+          t = tc[k];
+          best = q;
+          side = (uint32_t)k;
         }
-        best = q;
       }
     }
     cur = sp > 0 ? sn[(--sp) * kTraceBlock] : kDone;
@@ -3508,34 +3524,39 @@ k_ao_rays_sph(const srf_ray *__restrict__ primary, const srf_hit *__restrict__ h
   }
 }
 
+inline uint32_t max_nodes(const Accel *a) { return (uint32_t)(2 * a->n - 1); }
+inline bool small_tet(const Accel *a) { return !a->wide_stack && max_nodes(a) < (1u << 24); }
+
 // log2 of the rays a wavefront carries in a launch of n (wave_ray): the
-// fewest, 8 to 64, with which the launch has no more than `waves` wavefronts
-// (256 CUs hold 8,192 at 8 per SIMD). Measured with 64, 32, 16 and 8 (us):
+// fewest, 8 to 64, with which the launch has no more than `waves` wavefronts.
+inline uint32_t wave_rays(uint64_t n, uint64_t waves) {
+  uint32_t lg = 3;
+  while (lg < 6 && (n >> lg) > waves) lg++;
+  return lg;
+}
+// Measured with 64, 32, 16 and 8 (us):
 //   triangles   6k rays 380 223 174 161   83k 1470 1190 911 745
 //               262k 628 445 401 488   60k incoherent 184 162 153 171
 //   spheres     4k 1645 1140 700 506   197k 1535 1151 1213 1809
 //   hexahedra   14k 614 412 316 231   262k 1177 905 1020 1535
 //   lines       10k 763 437 284 195   77k 1015 741 681 880   320k 340 347 400 586
 // Triangle walks are the shortest, and twice the wavefronts still pay.
-// Rays that are traced one by one fill their wavefronts from 4,096 on.
-constexpr uint64_t kTriWaves = 16384, kWaves = 8192, kAloneWaves = 4096;
+// `alone`: rays without equal signs that a kernel traces one by one itself
+// share a wavefront from fewer on; the sphere and solid kernels leave them to
+// a second launch.
 constexpr WaveRays kFullWaves = {6u, 6u};
-inline WaveRays wave_rays(uint64_t n, uint64_t waves) {
-  WaveRays w = {3u, 3u};
-  while (w.lg < 6 && (n >> w.lg) > waves) w.lg++;
-  while (w.lg_alone < 6 && (n >> w.lg_alone) > kAloneWaves) w.lg_alone++;
-  if (w.lg_alone < w.lg) w.lg_alone = w.lg;
-  return w;
+inline WaveRays wave_rays(const Accel *a, uint64_t n) {
+  const uint32_t lg = wave_rays(n, a->kind == kTri ? 16384 : 8192);
+  if (a->kind == kSph || a->kind == kSol) return WaveRays{lg, lg};
+  return WaveRays{lg, std::max(lg, wave_rays(n, 4096))};
 }
 // blocks for n rays, carried as w says
 inline uint32_t trace_blocks(uint64_t n, WaveRays w = kFullWaves) {
   return xcd_grid(wave_run_blocks(n, w) << (w.lg_alone - w.lg));
 }
-inline uint32_t max_nodes(const Accel *a) { return (uint32_t)(2 * a->n - 1); }
 // every node index fits the 3-byte stack entries
 inline bool small_nodes(const Accel *a) { return !a->wide_stack && 2 * a->n - 1 <= (1u << 24); }
 // every node index fits the tetra kernel's 24-bit entries
-inline bool small_tet(const Accel *a) { return !a->wide_stack && max_nodes(a) < (1u << 24); }
 inline SphSub sph_sub(const Accel *a) {
   SphSub s{};
   if (a->kind == kSph && a->nbig) {
@@ -3553,7 +3574,7 @@ inline SphSub sph_sub(const Accel *a) {
 srf_status trace_tri(const Accel *a, const srf_ray *rays, uint64_t n, srf_hit *hits,
                      hipStream_t s) {
   if (n == 0) return SRF_OK;
-  const WaveRays lg = wave_rays(n, kTriWaves);
+  const WaveRays lg = wave_rays(a, n);
   if (small_nodes(a))
     hipLaunchKernelGGL((k_trace_tri_wave<true>), dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0, s,
                        (const float4 *)a->nodes, (const float4 *)a->prims, a->params, rays,
@@ -3569,7 +3590,7 @@ srf_status trace_tri(const Accel *a, const srf_ray *rays, uint64_t n, srf_hit *h
 srf_status trace_tet(const Accel *a, const srf_ray *rays, uint64_t n, const float *scalars,
                      srf_hit *hits, srf_tet_hit_ext *ext, hipStream_t s) {
   if (n == 0) return SRF_OK;
-  const WaveRays lg = wave_rays(n, kWaves);
+  const WaveRays lg = wave_rays(a, n);
   if (small_tet(a))
     hipLaunchKernelGGL((k_trace_tet<false, true>), dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0,
                        s, (const float4 *)a->nodes, (const float4 *)a->prims,
@@ -3610,7 +3631,7 @@ srf_status launch_sol(const Accel *a, const srf_ray *rays, uint64_t n, WaveRays 
 srf_status trace_lin(const Accel *a, const srf_ray *rays, uint64_t n, srf_hit *hits,
                      srf_line_hit_ext *ext, hipStream_t s) {
   if (n == 0) return SRF_OK;
-  const WaveRays lg = wave_rays(n, kWaves);
+  const WaveRays lg = wave_rays(a, n);
   hipLaunchKernelGGL(k_trace_lin<false>, dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0, s,
                      (const float4 *)a->nodes, (const float4 *)a->prims, a->params, rays,
                      (uint32_t)n, lg, hits, ext, nullptr, nullptr, max_nodes(a), (uint32_t)a->n,
@@ -3622,27 +3643,30 @@ srf_status trace_lin(const Accel *a, const srf_ray *rays, uint64_t n, srf_hit *h
 srf_status trace_sol(const Accel *a, const srf_ray *rays, uint64_t n, const float *scalars,
                      srf_hit *hits, srf_solid_hit_ext *ext, hipStream_t s) {
   if (n == 0) return SRF_OK;
-  const WaveRays lg = wave_rays(n, kWaves);
-  const srf_status st = launch_sol<1>(a, rays, n, lg, scalars, hits, ext, nullptr, nullptr, s);
+  const srf_status st = launch_sol<1>(a, rays, n, wave_rays(a, n), scalars, hits, ext, nullptr,
+                                      nullptr, s);
   if (st != SRF_OK) return st;
-  return launch_sol<2>(a, rays, n, lg, scalars, hits, ext, nullptr, nullptr, s);
+  return launch_sol<2>(a, rays, n, kFullWaves, scalars, hits, ext, nullptr, nullptr, s);
 }
 
 srf_status trace_sph(const Accel *a, const srf_ray *rays, const srf_sphere_prev *prev,
                      uint64_t n, srf_hit *hits, hipStream_t s) {
   if (n == 0) return SRF_OK;
-  const WaveRays lg = wave_rays(n, kWaves);
+  const WaveRays lg = wave_rays(a, n);
   // the wavefront traversal for groups of equal direction signs, then the
-  // per-lane one for the rest
+  // per-lane one for the rays it marked
   hipLaunchKernelGGL((k_trace_sph<false, 1>), dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0, s,
                      (const float4 *)a->nodes, (const float4 *)a->prims, a->sorted_index, rays,
                      prev, (uint32_t)n, hits, nullptr, nullptr, max_nodes(a), (uint32_t)a->n,
                      sph_sub(a), a->params, lg);
   SRF_HIP(hipGetLastError());
-  hipLaunchKernelGGL((k_trace_sph<false, 2>), dim3(trace_blocks(n, lg)), dim3(kTraceBlock), 0, s,
-                     (const float4 *)a->nodes, (const float4 *)a->prims, a->sorted_index, rays,
+  // (83k random rays on 2M spheres: 4.2 ms in wavefronts of 64, 3.3 in 32s)
+  const uint32_t lg2 = wave_rays(n, 3072);
+  const WaveRays alone = {lg2, lg2};
+  hipLaunchKernelGGL((k_trace_sph<false, 2>), dim3(trace_blocks(n, alone)), dim3(kTraceBlock), 0,
+                     s, (const float4 *)a->nodes, (const float4 *)a->prims, a->sorted_index, rays,
                      prev, (uint32_t)n, hits, nullptr, nullptr, max_nodes(a), (uint32_t)a->n,
-                     sph_sub(a), a->params, lg);
+                     sph_sub(a), a->params, alone);
   SRF_HIP(hipGetLastError());
   return SRF_OK;
 }

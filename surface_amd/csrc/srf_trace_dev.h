@@ -201,6 +201,23 @@ __device__ __forceinline__ bool wave_ray(const srf_ray *__restrict__ rays, uint3
   return true;
 }
 
+// A launch of wavefront walks leaves the rays it has no group for to a second
+// launch by a mark in their hits (no hit has a negative t), so that the two
+// can spread their rays over wavefronts each as it wants.
+constexpr float kAlone = -1.0f;
+__device__ __forceinline__ void leave_alone(srf_hit *__restrict__ hits, const WaveRay &r) {
+  if (r.own) hits[r.i].t = kAlone;
+}
+// The second launch's ray, 2^lg of a wavefront: false for a lane without one.
+__device__ __forceinline__ bool ray_alone(const srf_hit *__restrict__ hits, uint32_t n,
+                                          uint32_t lg, WaveRay &r) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint64_t i = ((uint64_t)(xcd_block() * (kTraceBlock / 64) + (threadIdx.x >> 6)) << lg) + lane;
+  r.i = (uint32_t)i;
+  r.first = r.own = true;
+  return (lane >> lg) == 0 && i < n && hits[i].t == kAlone;
+}
+
 // ------------------------------------------------------- wavefront groups
 //
 // A wavefront traversal (one walk for many lanes, nodes and primitives loaded

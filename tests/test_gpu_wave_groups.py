@@ -141,3 +141,23 @@ def test_launch_sizes_match_oracle(S, orc, kind, n):
         want = want[0] if isinstance(want, tuple) else want
         assert np.array_equal(got["prim_id"][check], want["prim_id"])
         assert np.array_equal(got["t"][check].view(np.uint32), want["t"].view(np.uint32))
+
+
+# spheres and solids mark the rays that no group takes in the hits themselves:
+# what the caller's buffer held before must not matter, nor a launch of none
+@pytest.mark.parametrize("kind", ["sph", "sol5", "sol6", "sol8"])
+def test_marks_in_the_hits_are_the_call_s_own(S, orc, kind):
+    import torch
+    geo, view, half = geometry(kind)
+    a, oracle = build(S, orc, kind, geo)
+    for name, rays in ray_sets(view, half).items():
+        want = oracle(rays)
+        want = want[0] if isinstance(want, tuple) else want
+        dev = S.device_tensor(rays)
+        for fill in (-1.0, float("nan"), 0.0):
+            hits = torch.full((len(rays) + 64, 4), fill, device="cuda")
+            got = S.hits_to_numpy(a.Traverse(dev, hits=hits)[:len(rays)].contiguous())
+            assert np.array_equal(got["prim_id"], want["prim_id"]), (name, fill)
+            assert np.array_equal(got["t"].view(np.uint32), want["t"].view(np.uint32))
+            tail = hits[len(rays):]
+            assert bool((torch.isnan(tail) if fill != fill else tail == fill).all())
