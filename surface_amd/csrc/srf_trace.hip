@@ -3534,21 +3534,41 @@ inline uint32_t wave_rays(uint64_t n, uint64_t waves) {
   while (lg < 6 && (n >> lg) > waves) lg++;
   return lg;
 }
-// Measured with 64, 32, 16 and 8 (us):
-//   triangles   6k rays 380 223 174 161   83k 1470 1190 911 745
-//               262k 628 445 401 488   60k incoherent 184 162 153 171
-//   spheres     4k 1645 1140 700 506   197k 1535 1151 1213 1809
-//   hexahedra   14k 614 412 316 231   262k 1177 905 1020 1535
-//   lines       10k 763 437 284 195   77k 1015 741 681 880   320k 340 347 400 586
-// Triangle walks are the shortest, and twice the wavefronts still pay.
+// How many wavefronts pay depends on what the rays of one share: little in a
+// tree whose leaves are smaller than the rays' spacing, nearly the whole walk
+// in a small tree. Camera frames, us with 64, 32, 16 and 8 rays:
+//   triangles   262k rays on 2k 50 76 94 142, on 32k 144 157 172 239, on 130k
+//               310 279 288 381, on 522k 683 547 540 721; 83k on 522k 841 674 567 537
+//   tetrahedra  83k on 3k 67 70 91 131, on 1.6M 426 333 350 369; 262k on 384k 190 244 358 612
+//   spheres     50k on 3k 223 210 156 167; 262k on 30k 196 263 379 607, on 16M
+//               5848 4243 4259 5424; 131k on 2M 1259 1006 996 1330
+//   hexahedra   131k on 14k 616 385 366 489, 262k 650 580 720 1075
+//   lines       262k on 197k 639 685 881 1350, 83k 812 582 582 620
 // `alone`: rays without equal signs that a kernel traces one by one itself
 // share a wavefront from fewer on; the sphere and solid kernels leave them to
 // a second launch.
 constexpr WaveRays kFullWaves = {6u, 6u};
 inline WaveRays wave_rays(const Accel *a, uint64_t n) {
-  const uint32_t lg = wave_rays(n, a->kind == kTri ? 16384 : 8192);
-  if (a->kind == kSph || a->kind == kSol) return WaveRays{lg, lg};
-  return WaveRays{lg, std::max(lg, wave_rays(n, 4096))};
+  uint32_t lg, alone;
+  switch (a->kind) {
+    case kTri:
+      lg = wave_rays(n, a->n < 65536 ? 4096 : 16384);
+      alone = std::max(lg, wave_rays(n, 4096));
+      break;
+    case kTet:  // (without the small stack every ray is traced by itself)
+      lg = alone = wave_rays(n, !small_tet(a) ? 3072 : a->n < 100000 ? 4096 : 5120);
+      break;
+    case kSph:
+      lg = alone = wave_rays(n, a->n < 100000 ? 5120 : 8192);
+      break;
+    case kLin:
+      lg = wave_rays(n, 8192);
+      alone = std::max(lg, wave_rays(n, 4096));
+      break;
+    default:  // solids
+      lg = alone = wave_rays(n, 8192);
+  }
+  return WaveRays{lg, alone};
 }
 // blocks for n rays, carried as w says
 inline uint32_t trace_blocks(uint64_t n, WaveRays w = kFullWaves) {
