@@ -1126,7 +1126,7 @@ k_trace_sph(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     }
   };
   if constexpr (kWavePath) {
-    const int group = wave_group(s, group_reach(params), ray.first);
+    const int group = wave_group(s, group_reach(params), ray.first, lg.singles != 0);
     walk_groups(group, walk);
     if (group == -1) leave_alone(hits, ray);
     if (group < 0) return;
@@ -2778,7 +2778,7 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     for (int k = 0; k < 3; k++)
       cext = fmaxf(cext, fmaxf(fabsf(P.root_bmin[k]), fabsf(P.root_bmax[k])));
     sol_frame(sq, s, cext);
-    const int group = wave_group(s, group_reach(params), ray.first);
+    const int group = wave_group(s, group_reach(params), ray.first, lg.singles != 0);
     walk_groups(group, walk);
     if (group == -1) leave_alone(hits, ray);
     if (group < 0) return;
@@ -3148,7 +3148,7 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   };
   if constexpr (!kAny) {
     queue_start(queue, s, prev);
-    const int g = wave_group(s, group_reach(params), ray.first);
+    const int g = wave_group(s, group_reach(params), ray.first, lg.singles != 0);
     walk_groups(g, walk);
     if (g != -1) cur = kDone;
     if (g >= 0) {
@@ -3547,9 +3547,9 @@ inline uint32_t wave_rays(uint64_t n, uint64_t waves) {
 // `alone`: rays without equal signs that a kernel traces one by one itself
 // share a wavefront from fewer on; the sphere and solid kernels leave them to
 // a second launch.
-constexpr WaveRays kFullWaves = {6u, 6u};
+constexpr WaveRays kFullWaves = {6u, 6u, 1u};
 inline WaveRays wave_rays(const Accel *a, uint64_t n) {
-  uint32_t lg, alone;
+  uint32_t lg, alone, singles = 1;
   switch (a->kind) {
     case kTri:
       lg = wave_rays(n, a->n < 65536 ? 4096 : 16384);
@@ -3560,15 +3560,17 @@ inline WaveRays wave_rays(const Accel *a, uint64_t n) {
       break;
     case kSph:
       lg = alone = wave_rays(n, a->n < 100000 ? 5120 : 8192);
+      singles = a->n >= 16384;
       break;
     case kLin:
       lg = wave_rays(n, 8192);
       alone = std::max(lg, wave_rays(n, 4096));
+      singles = a->n >= 32768;
       break;
     default:  // solids
       lg = alone = wave_rays(n, 8192);
   }
-  return WaveRays{lg, alone};
+  return WaveRays{lg, alone, singles};
 }
 // blocks for n rays, carried as w says
 inline uint32_t trace_blocks(uint64_t n, WaveRays w = kFullWaves) {
@@ -3682,7 +3684,7 @@ srf_status trace_sph(const Accel *a, const srf_ray *rays, const srf_sphere_prev 
   SRF_HIP(hipGetLastError());
   // (83k random rays on 2M spheres: 4.2 ms in wavefronts of 64, 3.3 in 32s)
   const uint32_t lg2 = wave_rays(n, 3072);
-  const WaveRays alone = {lg2, lg2};
+  const WaveRays alone = {lg2, lg2, 1u};
   hipLaunchKernelGGL((k_trace_sph<false, 2>), dim3(trace_blocks(n, alone)), dim3(kTraceBlock), 0,
                      s, (const float4 *)a->nodes, (const float4 *)a->prims, a->sorted_index, rays,
                      prev, (uint32_t)n, hits, nullptr, nullptr, max_nodes(a), (uint32_t)a->n,

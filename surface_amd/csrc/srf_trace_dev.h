@@ -149,6 +149,7 @@ __device__ __forceinline__ void boxes_plain(const RaySetup &s, uint32_t sb, floa
 // fourth CU: 450 us).
 struct WaveRays {
   uint32_t lg, lg_alone;  // lg <= lg_alone
+  uint32_t singles;       // whether lanes that share with none are worth a walk each
 };
 // blocks that one part of every run takes
 __host__ __device__ __forceinline__ uint32_t wave_run_blocks(uint64_t n, WaveRays w) {
@@ -260,25 +261,29 @@ __device__ __forceinline__ uint64_t next_group(const RaySetup &s, uint64_t todo,
 }
 
 // The number of this lane's group, -1 for a lane that is traced alone, -2 for
-// one that repeats another's ray (`first` false). Lanes of one sign are group 0. Up to kGroupTries groups are kept whatever their
-// sizes; where the lanes do not fit in so many, only groups of kGroupMin
-// lanes or more.
-__device__ __forceinline__ int wave_group(const RaySetup &s, float reach, bool first) {
+// one that repeats another's ray (`first` false). Lanes of one sign are group
+// 0. Up to kGroupTries groups are kept whatever their sizes; where the lanes
+// do not fit in so many, only groups of kGroupMin lanes or more, and where they
+// need more than half of them, no single lanes without `singles`.
+__device__ __forceinline__ int wave_group(const RaySetup &s, float reach, bool first,
+                                          bool singles) {
   const uint32_t sb = __builtin_amdgcn_readfirstlane(s.sbits);
   if (__all(s.sbits == sb)) return first ? 0 : -2;
   uint64_t todo = __ballot(first);
   const int lane = threadIdx.x & 63;
-  int group = -1, size = 0;
+  int group = -1, size = 0, groups = 0;
   for (int g = 0; g < kGroupTries && todo; g++) {
     const uint64_t m = next_group(s, todo, reach);
     todo &= ~m;
+    groups++;
     if ((m >> lane) & 1u) {
       group = g;
       size = __popcll(m);
     }
   }
   if (!first) return -2;
-  return todo && size < kGroupMin ? -1 : group;
+  const int least = todo ? kGroupMin : (groups > kGroupTries / 2 && !singles ? 2 : 1);
+  return size < least ? -1 : group;
 }
 
 // Calls walk(mask) (uniform control flow) for each group of a wavefront.
