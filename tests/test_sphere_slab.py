@@ -11,7 +11,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from test_sphere_pad import adversarial, f32, f64, sphere_test
+from test_sphere_pad import PAD, PAD_ORIGIN, adversarial, f32, f64, sphere_test
 
 FLT_MAX, FLT_MIN = np.finfo(f32).max, np.finfo(f32).tiny
 
@@ -26,7 +26,7 @@ def enters(o, d, lo_box, hi_box, t):
     with np.errstate(all="ignore"):
         far = np.maximum(np.abs(o - lo_box), np.abs(o - hi_box)).astype(f32)
         dist = np.sqrt((far * far).sum(1, dtype=f32))
-        pad = f32(9.6e-4) * dist + f32(4e-7) * np.abs(o).sum(1, dtype=f32)
+        pad = f32(PAD) * dist + f32(PAD_ORIGIN) * np.abs(o).sum(1, dtype=f32)
         a = (d * d).sum(1, dtype=f32)
         sign = d < 0
         mag = np.minimum(np.abs(f32(1) / d), f32(1e30))
