@@ -92,7 +92,7 @@ TRAFFIC = {
     "heightfield512": 174_836_000,
     "heightfield725": 359_670_000,
     "tetgrid64": 131_817_300,
-    "plummer16M_primary": 1_176_510_000,  # both launches
+    "plummer16M_primary": 1_112_760_000,  # both launches
     "scene64_upper": 23_603_015_759,      # persistent launch, 128-lane blocks
     "k_vol_fwd": 275_953_791,             # the march without checkpoints
     "k_vol_bwd": 1_376_455_261,

@@ -1528,9 +1528,6 @@ __device__ __forceinline__ Box merge_lr(const Box &l, const Box &r) {
   return m;
 }
 
-// One thread per leaf (global leaf id y): leaf box + packed primitives, the
-// leaf's own slot 0 and its parent's slot for it. With M the sorted index
-// comes from the shared scratch and is copied into the mesh's accelerator.
 // Notes a leaf box with an infinite or NaN bound (or bounds so large that
 // their sum overflows): the traversals' short box test is not for such trees.
 __device__ __forceinline__ void note_box(BuildParams *params, const Box &b) {
@@ -1539,6 +1536,9 @@ __device__ __forceinline__ void note_box(BuildParams *params, const Box &b) {
   if (!(sum <= FLT_MAX)) atomicOr(&params->odd_box, 1u);
 }
 
+// One thread per leaf (global leaf id y): leaf box + packed primitives, the
+// leaf's own slot 0 and its parent's slot for it. With M the sorted index
+// comes from the shared scratch and is copied into the mesh's accelerator.
 template <int K, bool M>
 __global__ void __launch_bounds__(256) k_leaves(uint32_t n_all, const uint32_t *sidx_all,
                                                NodeOut o, const uint32_t *total_leaves,

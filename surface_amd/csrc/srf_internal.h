@@ -67,9 +67,12 @@ constexpr uint32_t kXcds = 8;
 // triangles to imbalance). A smaller grid has shorter ones, the power of two
 // that gives each XCD four or more (with runs of 128 a grid below 1024 blocks
 // left XCDs idle and one just above loads some twice: 512^2 rays through a
-// 128^3 volume, march and adjoint, 2360 -> 1741 us), but not below 32, a block
-// for each CU of an XCD: a handful of blocks share the loads into one L2
-// (2,013 rays on 8k triangles: 106 us on one XCD, 111 us over eight). The
+// 128^3 volume, march and adjoint, 2360 -> 1741 us; 160^3 and 700x500 rays
+// 1854 -> 1563 us). Occlusion frames, which want the longer runs, lose to it
+// where one long run an XCD fits (131k rays on 522k triangles 722 -> 805 us,
+// 20k on 384k tetrahedra gain, 442 -> 356 us); one run an XCD instead of four
+// gives those back and the volumes' gain with them. Not below 32, a block for
+// each CU of an XCD (8 and 16 within 2 % at 300 to 20,000 rays). The
 // blocks after the last full set of runs keep their numbers, so the
 // renumbering is a bijection for any grid; xcd_grid fills the smallest up to
 // one set (kernels leave blocks without work at once).

@@ -255,8 +255,9 @@ template <uint32_t SB>
 __device__ __forceinline__ void tri_wave_closest(const float4 *__restrict__ nodes,
                                               const float4 *__restrict__ prims,
                                               uint32_t max_nodes, uint32_t nprims,
-                                              const RaySetup &s, uint32_t sbits, bool ds, float kEPS,
-                                              uint32_t prev, uint64_t mask, TriPairs &pairs,
+                                              const RaySetup &s, uint32_t sbits, bool ds,
+                                              float kEPS, uint32_t prev, uint64_t mask,
+                                              TriPairs &pairs,
                                               uint32_t *wnode, uint64_t *wmask, float &t, float &u,
                                               float &v, uint32_t &prim) {
   const uint32_t sb = SB < 8 ? SB : sbits;
@@ -1500,13 +1501,14 @@ __device__ __forceinline__ bool box_span(const RaySetup &s, float bx0, float by0
 
 // kSmall (node indices below 2^24): the stack in 16-bit planes, 6 bytes an
 // entry, so that the LDS holds 4 wavefronts per SIMD; the register cap of 4
-// wavefronts per SIMD (128 VGPRs, the closest-hit kernel spills 4) lets
+// wavefronts per SIMD (128 VGPRs, the closest-hit kernel spills 8) lets
 // them run (1024^2 rays on the 64^3 tetra grid: 0.53 -> 0.47 ms at 3 -> 4).
 template <bool kAny, bool kSmall>
 __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4)))
 k_trace_tet(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
             const uint4 *__restrict__ sorted_faces, const BuildParams *__restrict__ params,
-            const srf_ray *__restrict__ rays, uint32_t n, WaveRays lg, const float *__restrict__ scalars,
+            const srf_ray *__restrict__ rays, uint32_t n, WaveRays lg,
+            const float *__restrict__ scalars,
             srf_hit *__restrict__ hits, srf_tet_hit_ext *__restrict__ ext,
             const float *__restrict__ tmax_in, uint32_t *__restrict__ occluded,
             uint32_t max_nodes, uint32_t nprims) {
@@ -2602,9 +2604,11 @@ __device__ __attribute__((noinline)) SolCross sol_cross(const float4 *P, float o
 
 // kPart: 0 occlusion, a lane a ray; closest hits in two launches, 1 the groups
 // that share direction signs, 2 the rays that part 1 marked (leave_alone), a
-// lane a ray in full wavefronts. A lane's own walk has the FP64 test inline, without a register cap (pyramids
-// at 4 wavefronts per SIMD, 14 VGPRs spilled): with the call at every solid it
-// is 1.3 to 2.7 times as slow.
+// lane a ray in full wavefronts. A lane's own walk has the FP64 test inline,
+// without a register cap (pyramids at 4 wavefronts per SIMD, 16 VGPRs
+// spilled): with the call at every solid it is 1.2 to 2.7 times as slow (24^3
+// hexahedra, 1024^2 rays, occlusion 7.0 -> 2.6 ms; 262k random rays, closest
+// 5.5 -> 2.3 ms, prisms 4.4 -> 3.1, pyramids 5.2 -> 4.2).
 template <int NV, int kPart>
 __global__ void __launch_bounds__(kTraceBlock)
     __attribute__((amdgpu_waves_per_eu(NV == 5 ? 4 : kPart == 1 ? 3 : 1)))
@@ -2709,8 +2713,8 @@ k_trace_sol(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     // Closest hit once per group of lanes that share direction signs:
     // boxes are culled by entry alone, so a ray's visits do not depend on
     // its running hit and every lane's pre-order is one static order (the
-    // line kernel's shared-stack walk); each lane tests its own leaves'
-    // solids in its own order, the solids loaded through the scalar unit.
+    // line kernel's shared-stack walk). A leaf's solids are queued for the
+    // lanes that reach it, a ray's in its own order.
     const uint32_t sb = __builtin_amdgcn_readlane((int)s.sbits, __builtin_ctzll(group));
     const int wv = threadIdx.x >> 6;
     const uint64_t me = 1ull << (threadIdx.x & 63u);
@@ -3031,8 +3035,8 @@ __device__ __forceinline__ bool line_isect(float &t, float &u, float &v, bool &h
 template <bool kAny>
 __global__ void __launch_bounds__(kTraceBlock)
 k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
-            const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays, uint32_t n, WaveRays lg,
-            srf_hit *__restrict__ hits, srf_line_hit_ext *__restrict__ ext,
+            const BuildParams *__restrict__ params, const srf_ray *__restrict__ rays, uint32_t n,
+            WaveRays lg, srf_hit *__restrict__ hits, srf_line_hit_ext *__restrict__ ext,
             const float *__restrict__ tmax_in, uint32_t *__restrict__ occluded, uint32_t max_nodes,
             uint32_t nprims, uint32_t cap) {
   // a wavefront needs the queue's space or its lanes' stacks, never both
@@ -3077,13 +3081,14 @@ k_trace_lin(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
     return hit;
   };
   auto walk = [&](uint64_t group) {
-    // Closest hit once per group of lanes that share direction signs. A node's boxes are culled by entry alone (no distance), so the nodes a
+    // Closest hit once per group of lanes that share direction signs. A
+    // node's boxes are culled by entry alone (no distance), so the nodes a
     // ray visits do not depend on its running hit, and with shared signs
     // every lane's pre-order (near child by the split axis' sign, far child
     // pushed when both boxes are entered) is one static order: the
     // wavefront walks the union of the lanes' visits in that order with one
-    // stack of (node, lane mask), and each lane tests its own leaves' lines
-    // in its own order, as in the per-ray loop below.
+    // stack of (node, lane mask), and queues each leaf's lines for the lanes
+    // that reach it, a ray's in the order of the per-ray loop below.
     const uint32_t sb = __builtin_amdgcn_readlane((int)s.sbits, __builtin_ctzll(group));
     const int wv = threadIdx.x >> 6;
     const uint64_t me = 1ull << (threadIdx.x & 63u);

@@ -213,7 +213,8 @@ __device__ __forceinline__ void leave_alone(srf_hit *__restrict__ hits, const Wa
 __device__ __forceinline__ bool ray_alone(const srf_hit *__restrict__ hits, uint32_t n,
                                           uint32_t lg, WaveRay &r) {
   const uint32_t lane = threadIdx.x & 63u;
-  const uint64_t i = ((uint64_t)(xcd_block() * (kTraceBlock / 64) + (threadIdx.x >> 6)) << lg) + lane;
+  const uint32_t wave = xcd_block() * (kTraceBlock / 64) + (threadIdx.x >> 6);
+  const uint64_t i = ((uint64_t)wave << lg) + lane;
   r.i = (uint32_t)i;
   r.first = r.own = true;
   return (lane >> lg) == 0 && i < n && hits[i].t == kAlone;

@@ -115,8 +115,9 @@ def test_mixed_sign_wavefronts_match_oracle(S, orc, kind):
 
 
 # launches that carry 8, 16, 32 and 64 rays per wavefront, coherent and not
-# (random rays of one wavefront stay together from 262,144 / 64 runs on), at
-# sizes around a run of 64 and a block
+# (random rays that a kernel traces one by one itself share wavefronts of 32
+# from 65,552 and of 64 from 131,104 rays on), at sizes around a run of 64 and a
+# block
 @pytest.mark.parametrize("kind", ["tri", "sph", "lin", "tet", "sol8"])
 @pytest.mark.parametrize("n", [1, 63, 65, 127, 129, 40_007, 150_001, 280_000])
 def test_launch_sizes_match_oracle(S, orc, kind, n):
