@@ -162,3 +162,33 @@ def test_marks_in_the_hits_are_the_call_s_own(S, orc, kind):
             assert np.array_equal(got["t"].view(np.uint32), want["t"].view(np.uint32))
             tail = hits[len(rays):]
             assert bool((torch.isnan(tail) if fill != fill else tail == fill).all())
+
+
+@pytest.mark.parametrize("kind", ["sph", "sol8"])
+def test_two_launch_traces_in_a_graph(S, orc, kind):
+    # rays in groups, lone ones and both mixed take turns in one captured call
+    import torch
+    geo, view, half = geometry(kind)
+    a, oracle = build(S, orc, kind, geo)
+    sets = [r[:1500] for r in ray_sets(view, half).values()]
+    rays = S.device_tensor(sets[0]).clone()
+    hits = torch.empty((len(rays), 4), device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        a.Traverse(rays, hits=hits)
+    torch.cuda.current_stream().wait_stream(side)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        a.Traverse(rays, hits=hits)
+    for r in sets + sets[::-1]:
+        rays.copy_(S.device_tensor(np.ascontiguousarray(r)))
+        g.replay()
+        torch.cuda.synchronize()
+        got = S.hits_to_numpy(hits)
+        eager = S.hits_to_numpy(a.Traverse(rays))
+        want = oracle(np.ascontiguousarray(r))
+        want = want[0] if isinstance(want, tuple) else want
+        assert np.array_equal(got["prim_id"], want["prim_id"])
+        assert np.array_equal(got["t"].view(np.uint32), want["t"].view(np.uint32))
+        assert got.tobytes() == eager.tobytes()
