@@ -68,12 +68,12 @@ constexpr uint32_t kXcds = 8;
 // that gives each XCD four or more (with runs of 128 a grid below 1024 blocks
 // left XCDs idle and one just above loads some twice: 512^2 rays through a
 // 128^3 volume, march and adjoint, 2360 -> 1741 us; 160^3 and 700x500 rays
-// 1854 -> 1563 us). Occlusion frames, which want the longer runs, lose to it
-// where one long run an XCD fits (131k rays on 522k triangles 722 -> 805 us,
-// 20k on 384k tetrahedra gain, 442 -> 356 us); one run an XCD instead of four
-// gives those back and the volumes' gain with them. Not below 32, a block for
-// each CU of an XCD (8 and 16 within 2 % at 300 to 20,000 rays). The
-// blocks after the last full set of runs keep their numbers, so the
+// 1854 -> 1563 us). Occlusion of triangles and tetrahedra, whose frames are
+// more even, wants the longer runs and has one an XCD (kRuns; 131k rays on 522k
+// triangles 805 us in four, 723 in one); the volumes' gain goes with it (512^2
+// rays 1327 -> 1721 us), other traversals are within 2 % either way. Not below
+// 32, a block for each CU of an XCD (8 and 16 within 2 % at 300 to 20,000 rays).
+// The blocks after the last full set of runs keep their numbers, so the
 // renumbering is a bijection for any grid; xcd_grid fills the smallest up to
 // one set (kernels leave blocks without work at once).
 constexpr uint32_t kXcdRunMin = 5, kXcdRunMax = 7;  // log2
@@ -81,8 +81,9 @@ __host__ __device__ __forceinline__ uint32_t xcd_grid(uint32_t blocks) {
   const uint32_t set = kXcds << kXcdRunMin;
   return blocks < set ? set : blocks;
 }
+template <uint32_t kRuns = 4>
 __device__ __forceinline__ uint32_t xcd_block() {
-  const uint32_t per = gridDim.x / (4 * kXcds);
+  const uint32_t per = gridDim.x / (kRuns * kXcds);
   const uint32_t lg = per >> kXcdRunMax ? kXcdRunMax : (per >> kXcdRunMin ? 31 - __builtin_clz(per)
                                                                         : kXcdRunMin);
   const uint32_t set = kXcds << lg, b = blockIdx.x;

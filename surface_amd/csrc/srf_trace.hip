@@ -66,7 +66,7 @@ k_trace_tri(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   __shared__ uint8_t stack_hi[kSmall ? kTraceStack * kTraceBlock : 1];
   __shared__ uint32_t wnode[kAny ? kTraceBlock / 64 : 1][kTraceStack];
   __shared__ uint64_t wmask[kAny ? kTraceBlock / 64 : 1][kTraceStack];
-  const uint32_t i = xcd_block() * kTraceBlock + threadIdx.x;
+  const uint32_t i = xcd_block<1>() * kTraceBlock + threadIdx.x;
   if (i >= n) return;
   uint32_t flags, prev;
   const RaySetup s = setup_ray(rays, i, flags, prev);
@@ -1544,7 +1544,7 @@ k_trace_tet(const float4 *__restrict__ nodes, const float4 *__restrict__ prims,
   __shared__ uint32_t wv_par[kSmall ? kTraceBlock / 64 : 1][kTraceStack];
   __shared__ uint64_t wv_msk[kSmall ? kTraceBlock / 64 : 1][kTraceStack];
   WaveRay ray;
-  if (!wave_ray(rays, n, lg, ray)) return;
+  if (!wave_ray<kAny ? 1 : 4>(rays, n, lg, ray)) return;
   if (!ray.own) return;
   const uint32_t i = ray.i;
   uint32_t flags, prev;

@@ -164,11 +164,12 @@ struct WaveRay {
 // False for a wavefront without rays. The lanes beyond the wavefront's rays,
 // and the last one's beyond n, repeat a ray: the paired and queued leaf tests
 // want all 64 lanes.
+template <uint32_t kRuns = 4>
 __device__ __forceinline__ bool wave_ray(const srf_ray *__restrict__ rays, uint32_t n, WaveRays w,
                                          WaveRay &r) {
   const uint32_t lane = threadIdx.x & 63u;
   uint32_t lg = w.lg;
-  uint32_t block = xcd_block(), part_no = 0;
+  uint32_t block = xcd_block<kRuns>(), part_no = 0;
   const uint32_t lg_parts = w.lg_alone - lg;
   const uint32_t run_blocks = wave_run_blocks(n, w);
   for (; part_no < (1u << lg_parts) && block >= run_blocks; part_no++) block -= run_blocks;
